@@ -10,7 +10,7 @@ block, TRSM and Schur-update launches spread over the GPU).
 - `CostModel` is the library's 8 -> 64 -> 64 -> 2 FP32 MLP, trained on the
   device (`sylver_amd_mlp_train`) on the autotuner's timings, predicting
   log2 of the time of both variants from eight shape features; its choice
-  is the variant with the smaller prediction.
+  is the variant with the smaller prediction where the two differ clearly.
 - `choose_variants` turns either into the per-front variant array of
   `set_front_variants`. Fronts outside [M_MIN, M_MAX] rows keep the default
   rule (the one-workgroup kernel below, the tiled path above), where one
@@ -23,6 +23,12 @@ import math
 import numpy as np
 
 M_MIN, M_MAX = 32, 2048  # rows of the fronts whose variant is chosen
+DEFAULT_MAX = 256  # the default rule: one workgroup up to this many rows
+# log2 of the predicted ratio of the two times below which the default rule
+# stands: the model's error on a held-out front (root mean square 0.13-0.17)
+# is larger than such a gain, and near the crossover a wrong choice costs more
+# than a right one brings
+MARGIN = 0.15
 
 
 def node_flops(m, n):
@@ -126,5 +132,9 @@ class CostModel:
         return self.S.mlp_predict(self.params, x)
 
     def pick_one_wg(self, x):
+        """The variant with the smaller prediction, or the default rule's where
+        the two are within MARGIN of each other."""
         p = self.predict(x)
-        return p[:, 0] < p[:, 1]
+        gain = p[:, 1] - p[:, 0]
+        one_wg = np.exp2(np.asarray(x)[:, 0].astype(np.float64)) <= DEFAULT_MAX + 0.5
+        return np.where(np.abs(gain) > MARGIN, gain > 0, one_wg)

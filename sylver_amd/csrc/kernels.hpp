@@ -95,6 +95,24 @@ __device__ inline void buf_store(__amdgpu_buffer_rsrc_t r, uint32_t off, double 
    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2, v), r, (int)off, 0, 0);
 }
 
+// v, the same in every lane, as a scalar: a buffer access whose scalar offset
+// the compiler holds in a vector register becomes a loop over the lanes.
+__device__ __forceinline__ uint32_t uniform(uint32_t v) { return __builtin_amdgcn_readfirstlane((int)v); }
+// The same with a scalar part of the offset (uniform over the wave).
+__device__ inline float buf_load_s(__amdgpu_buffer_rsrc_t r, uint32_t off, uint32_t soff, float*) {
+   return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, (int)off, (int)soff, 0));
+}
+__device__ inline double buf_load_s(__amdgpu_buffer_rsrc_t r, uint32_t off, uint32_t soff, double*) {
+   return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, (int)off, (int)soff, 0));
+}
+__device__ inline void buf_store_s(__amdgpu_buffer_rsrc_t r, uint32_t off, uint32_t soff, float v) {
+   __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned int, v), r, (int)off, (int)soff, 0);
+}
+__device__ inline void buf_store_s(__amdgpu_buffer_rsrc_t r, uint32_t off, uint32_t soff, double v) {
+   typedef unsigned int u2 __attribute__((ext_vector_type(2)));
+   __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2, v), r, (int)off, (int)soff, 0);
+}
+
 typedef double v4d __attribute__((ext_vector_type(4)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 
@@ -423,14 +441,50 @@ __device__ inline typename Mfma<T>::acc_t lds_mma16(const T* A, int lda, const T
    return acc;
 }
 
+// The elimination of a 16-column panel held a row per lane (lanes 0..15 the
+// diagonal block's rows): column step j forms l_ij = a_ij / sqrt(d) and
+// a_ic -= (l_ij / sqrt(d)) a_cj for c > j, a_cj broadcast from lane c by
+// v_readlane. Branch-free, so the whole panel is one block the compiler can
+// schedule: the next pivot (row j + 1's update, then its broadcast) is formed
+// first and its reciprocal square root overlaps the rest of step j. Entries
+// above the diagonal may hold anything, no other lane reads them. After a
+// non-positive pivot the steps go on with meaningless values; the first such
+// column (1-based; 0: none) is what is returned: its diagonal entry of L is
+// not a number.
+template <typename T>
+__device__ __forceinline__ int panel_cholesky16(T (&r)[16], int lane) {
+   bool any = false;
+   T d = lane_bcast(r[0], 0);
+#pragma unroll
+   for (int j = 0; j < 16; ++j) {
+      T col[16];
+#pragma unroll
+      for (int c = j + 1; c < 16; ++c) col[c] = lane_bcast(r[j], c);
+      any |= !(d > T(0));
+      const T inv = rsqrt_nr(d);
+      r[j] *= inv;  // lane j holds d itself: d / sqrt(d)
+      const T t = r[j] * inv;
+      if (j + 1 < 16) {
+         r[j + 1] = fma(-t, col[j + 1], r[j + 1]);
+         d = lane_bcast(r[j + 1], j + 1);
+      }
+#pragma unroll
+      for (int c = j + 2; c < 16; ++c) r[c] = fma(-t, col[c], r[c]);
+   }
+   if (!any) return 0;
+   T l = T(1);
+   asm volatile("" : "+v"(lane));
+#pragma unroll
+   for (int c = 0; c < 16; ++c) l = lane == c ? r[c] : l;
+   return __builtin_ffsll(__ballot(!(l > T(0))));
+}
+
 // Cholesky of a 16-column panel in LDS by one wave: lanes 0..15 hold the
 // rows of the diagonal block, lanes 16..63 48 rows below it (rows o + 16 +
 // 48 w + ...; w = the wave's index among the panel's waves), each row in
-// registers. Column step j: l_ij = a_ij / sqrt(d), a_ic -= (l_ij / sqrt(d))
-// a_cj for c > j -- one FMA per element with a_cj broadcast from lane c by
-// v_readlane, so a step waits on no memory round trip. The rows below the
-// diagonal block are simply more rows of the same elimination, so a panel
-// of up to 64 rows takes the time of the 16x16 block alone. Every wave
+// registers (panel_cholesky16), so a step waits on no memory round trip. The
+// rows below the diagonal block are simply more rows of the same elimination,
+// so a panel of up to 64 rows takes the time of the 16x16 block alone. Every wave
 // of a panel factors the diagonal block (the same values, the same
 // operations, so the same results); wave 0 stores it.
 template <typename T, int LD>
@@ -441,30 +495,7 @@ __device__ __forceinline__ int wave_panel16(T* L, int o, int kb16, int w) {
    T r[16];
 #pragma unroll
    for (int c = 0; c < 16; ++c) r[c] = (live && (lane >= 16 || c <= lane)) ? L[row + (o + c) * LD] : T(0);
-   // Branch-free, so the whole panel is one block the compiler can schedule:
-   // the next pivot (row j + 1's update, then its broadcast) is formed first
-   // and its reciprocal square root overlaps the rest of step j. After a
-   // non-positive pivot the steps go on with meaningless values; the first
-   // such column is what is returned.
-   int bad = 0;
-   T d = lane_bcast(r[0], 0);
-#pragma unroll
-   for (int j = 0; j < 16; ++j) {
-      T col[16];
-#pragma unroll
-      for (int c = j + 1; c < 16; ++c) col[c] = lane_bcast(r[j], c);
-      bad = (bad == 0 && !(d > T(0))) ? j + 1 : bad;
-      const T inv = rsqrt_nr(d);
-      const T lj = r[j] * inv;
-      const T t = lj * inv;
-      r[j] = (lane == j) ? d * inv : lj;
-      if (j + 1 < 16) {
-         r[j + 1] = fma(-t, col[j + 1], r[j + 1]);
-         d = lane_bcast(r[j + 1], j + 1);
-      }
-#pragma unroll
-      for (int c = j + 2; c < 16; ++c) r[c] = fma(-t, col[c], r[c]);
-   }
+   const int bad = panel_cholesky16(r, lane);
    if (live) {
       if (lane < 16) {
          if (w == 0)
@@ -561,35 +592,77 @@ __device__ __forceinline__ int lds_potrf_panels(T* L, int kb16, int* sh_bad) {
    return *sh_bad;
 }
 
-// Blocked in-place inverse of the padded lower triangular kb16 x kb16 block
-// (block columns right to left; Tmp holds kNB x 16 elements, ld kNB).
+// Inverse of the padded lower triangular kb16 x kb16 block in LDS, written to
+// `out` (lower, ld kb) and transposed to `outT`, zeros in the other triangle.
+// The rows of inv(L)^T are the rows of I L^{-T}: each wave takes whole block
+// rows j of them and carries them through the substitution of k_strip,
+// X_b = -(sum_{k<b} X_k L_bk^T) inv(L_bb)^T for b > j from X_j =
+// inv(L_jj)^T, in registers and in k_strip's layout (item v of lane l is
+// X[l % 16][row(l, v)]). The block rows do not depend on one another, so one
+// barrier (after the 16 x 16 inverses) replaces the two per block column of
+// an inverse formed column by column in LDS (the launch that forms the
+// inverses of small fronts 28 -> 18 us); block rows j and 7 - j share a wave
+// to even out the work. The off-diagonal blocks of L are left as they
+// are. Tmp: a 16 x 17 tile per wave, through which `out` is stored by columns.
 template <typename T, int LD>
-__device__ void lds_trtri_blocked(T* L, T* Tmp, int kb16) {
+__device__ __forceinline__ void lds_trtri_store(T* L, T* Tmp, int kb, int kb16, T* __restrict__ out,
+                                                T* __restrict__ outT) {
    typedef typename Mfma<T>::acc_t acc_t;
-   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+   const int r = lane & 15, lq = lane >> 4;
    const int nbk = kb16 / 16;
+   T* tile = Tmp + wave * (16 * 17);
    for (int b = wave; b < nbk; b += 4) wave_trtri16<T, LD>(L + b * 16 + b * 16 * LD);
    __syncthreads();
-   for (int j = nbk - 2; j >= 0; --j) {
-      // T_i = sum_{k=j+1..i} X_ik L_kj for the block rows below j
-      for (int i = j + 1 + wave; i < nbk; i += 4) {
-         acc_t acc = acc_t{0, 0, 0, 0};
-         for (int k = j + 1; k <= i; ++k)
-            acc = lds_mma16<T, false>(L + i * 16 + k * 16 * LD, LD, L + k * 16 + j * 16 * LD, LD, acc);
+   for (int half = 0; half < 2; ++half) {
+      const int j = half ? 7 - wave : wave;
+      if (j >= nbk) continue;
+      const int i = j * 16 + r;  // the lane's row of inv(L)^T
+      T x[8][4];
 #pragma unroll
-         for (int v = 0; v < 4; ++v)
-            Tmp[(i * 16 + Mfma<T>::row(lane, v)) + (lane & 15) * kNB] = acc[v];
-      }
-      __syncthreads();
-      // X_ij = -T_i X_jj
-      for (int i = j + 1 + wave; i < nbk; i += 4) {
-         acc_t acc = acc_t{0, 0, 0, 0};
-         acc = lds_mma16<T, false>(Tmp + i * 16, kNB, L + j * 16 + j * 16 * LD, LD, acc);
+      for (int b = 0; b < 8; ++b) {
+         if (b < nbk) {
+            if (b < j) {
 #pragma unroll
-         for (int v = 0; v < 4; ++v)
-            L[(i * 16 + Mfma<T>::row(lane, v)) + (j * 16 + (lane & 15)) * LD] = -acc[v];
+               for (int v = 0; v < 4; ++v) x[b][v] = T(0);
+            } else if (b == j) {
+#pragma unroll
+               for (int v = 0; v < 4; ++v) x[b][v] = L[(b * 16 + Mfma<T>::row(lane, v)) + i * LD];
+            } else {
+               acc_t acc = acc_t{0, 0, 0, 0};
+#pragma unroll
+               for (int k = 0; k < b; ++k)
+                  if (k >= j)
+#pragma unroll
+                     for (int s = 0; s < 4; ++s)
+                        acc = Mfma<T>::op(L[(b * 16 + r) + (k * 16 + Mfma<T>::row(lane, s)) * LD], x[k][s], acc);
+               T tb[4];
+#pragma unroll
+               for (int v = 0; v < 4; ++v) tb[v] = -acc[v];
+               acc = acc_t{0, 0, 0, 0};
+#pragma unroll
+               for (int s = 0; s < 4; ++s)
+                  acc = Mfma<T>::op(L[(b * 16 + r) + (b * 16 + Mfma<T>::row(lane, s)) * LD], tb[s], acc);
+#pragma unroll
+               for (int v = 0; v < 4; ++v) x[b][v] = acc[v];
+            }
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+               const int c = b * 16 + Mfma<T>::row(lane, v);
+               if (i < kb && c < kb) outT[i + c * kb] = x[b][v];
+               tile[Mfma<T>::row(lane, v) * 17 + r] = x[b][v];
+            }
+            __builtin_amdgcn_wave_barrier();
+            // lane l: row r of the block b of inv(L), columns j * 16 + l / 16 + 4 v
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+               const int c = b * 16 + r, col = lq + 4 * v;
+               const T w = tile[r * 17 + col];
+               if (c < kb && j * 16 + col < kb) out[c + (j * 16 + col) * kb] = w;
+            }
+            __builtin_amdgcn_wave_barrier();
+         }
       }
-      __syncthreads();
    }
 }
 
@@ -677,35 +750,10 @@ __device__ void diag_block(const DiagTask& t, const NodeDesc& nd, T* __restrict_
          }
       }
       if (NOINV) return;
+      __syncthreads();  // every wave has read the factor; its diagonal blocks are inverted in place
    }
-   lds_trtri_blocked<T, LD>(L, Tmp, kb16);
-   T* out = dinv + nd.dinv_off + (int64_t)(t.k0 / kNB) * kNB * kNB;
-   T* outT = dinvT + nd.dinv_off + (int64_t)(t.k0 / kNB) * kNB * kNB;
-   if (kb == kNB) {
-      // row index from the low bits, stores coalesced per column (ld kb =
-      // kNB); LDS reads batched ahead of the stores as above
-      for (int e0 = 0; e0 < kNB * kNB; e0 += 8 * kThreads) {
-         T v[8], w[8];
-#pragma unroll
-         for (int u = 0; u < 8; ++u) {
-            const int e = e0 + u * kThreads + threadIdx.x, i = e & (kNB - 1), j = e >> 7;
-            v[u] = L[i + j * LD];
-            w[u] = L[j + i * LD];
-         }
-#pragma unroll
-         for (int u = 0; u < 8; ++u) {
-            const int e = e0 + u * kThreads + threadIdx.x, i = e & (kNB - 1), j = e >> 7;
-            out[e] = (i >= j) ? v[u] : T(0);
-            outT[e] = (j >= i) ? w[u] : T(0);
-         }
-      }
-   } else {
-      for (int e = threadIdx.x; e < kb * kb; e += kThreads) {
-         const int i = e % kb, j = e / kb;
-         out[i + j * kb] = (i >= j) ? L[i + j * LD] : T(0);
-         outT[i + j * kb] = (j >= i) ? L[j + i * LD] : T(0);
-      }
-   }
+   lds_trtri_store<T, LD>(L, Tmp, kb, kb16, dinv + nd.dinv_off + (int64_t)(t.k0 / kNB) * kNB * kNB,
+                          dinvT + nd.dinv_off + (int64_t)(t.k0 / kNB) * kNB * kNB);
 }
 
 template <typename T>
@@ -716,7 +764,7 @@ __global__ __launch_bounds__(kThreads) void k_diag(const DiagTask* __restrict__ 
                                                    int do_potrf) {
    constexpr int LD = kNB + 1;
    __shared__ T L[kNB * LD];
-   __shared__ T Tmp[kNB * 16];
+   __shared__ T Tmp[4 * 16 * 17];
    __shared__ int sh_bad;
    // the diagonal blocks are the factorization's critical path: their waves
    // win instruction issue over the look-ahead updates sharing the CU
@@ -759,7 +807,7 @@ static __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_num_vgpr(104
 // workgroup per 64 rows [r0, r0 + 64) below the diagonal block computes
 // X = A21 L11^{-T} by blocked substitution over 16-column blocks b,
 // X_b = (A_b - sum_{k<b} X_k L_bk^T) inv(L_bb)^T, with the 16x16 inverses
-// formed here from L11 (by wave_trtri16, as k_diag forms them). The chain
+// formed here from L11 (by wave_trtri16, as k_diag does). The chain
 // DIAG -> TRSM thus does not wait for the inverse of the whole block (formed
 // for the solves by the factorization's last launch).
 // Each wave owns 16 rows and keeps its 16x16 blocks in registers in the
@@ -1132,145 +1180,305 @@ static __global__ __launch_bounds__(kThreads) void k_update_bf16(const GemmTask*
 
 // ---------------------------------------------------------------------------
 // One workgroup factorizes a whole front (partial Cholesky over its first n
-// columns, Schur complement into the CB), right-looking in panels of kPB
-// columns. Per panel: the diagonal block in LDS (the blocked Cholesky and
-// inverse of the large-front diagonal kernel), the rows below as one product
-// with that inverse (L21 = A21 inv(L11)^T, 16-row strips on MFMA), then the
-// trailing lower triangle -= L21 L21^T on MFMA in 32 x 32 tiles with the
-// panel read through L1/L2: every trailing entry is read and written once
-// per panel, n / kPB passes in all.
+// columns, Schur complement into the CB), left-looking in panels of 16
+// columns: a panel is read once, receives the products of all columns before
+// it in one MFMA sum, is factored and written once; the contribution block
+// receives all n columns in one sum at the end. (The right-looking form with
+// 64-column panels before this one read and wrote the trailing block n / 64
+// times and inverted every 64 x 64 diagonal block for its panel solve; here
+// the rows below a diagonal block are rows of the same elimination, 16 + 48
+// to a wave, so there is no inverse and no separate solve.)
+// Bound: for a single front the panel chain -- per panel about 1 us of
+// elimination in FP64 (0.8 us FP32), the rest loads, the transposition
+// through LDS and two barriers; batched, the FP64 MFMA rate of the products.
+// Eight waves in 128 registers, so that two workgroups share a CU (four waves
+// in 256 left one per CU in FP64). Measured, before -> now: one front of 64
+// rows, 64 pivots 30.4 -> 16.7 us FP64, 26.7 -> 13.4 us FP32; 192 rows, 192
+// pivots 122 -> 73 us, 95 -> 51 us; 2048 fronts of 256 rows, 128 pivots 1373
+// -> 546 us (7.3 -> 18.4 TFLOP/s) FP64, 557 -> 317 us FP32.
 // Restates factor_front_posdef's arithmetic (reference src/factor.hxx:19-148,
 // src/kernels/factor.hxx:34-263) with a different blocking.
 // ---------------------------------------------------------------------------
-constexpr int kPB = 64;
+constexpr int kFrontThreads = 512;
 
+// Column window of a front for 32-bit addressing: element (row, c) of the
+// columns from `col` on is at byte (row + c ld) sizeof(T); the row part goes
+// in the lane's offset, the column part in the scalar one. A window serves
+// the 32 columns after its base, so any front size is reached. kOffMask as
+// the lane's offset masks the access (loads zero, stores nothing).
+constexpr uint32_t kOffMask = 0xFFFFFFFFu;
 template <typename T>
-__device__ void front_potrf_block(const NodeDesc& nd, T* __restrict__ F, int* info_slot) {
-   constexpr int LD = kPB + 1;
-   __shared__ T D[kPB * LD];
-   __shared__ T Tmp[kNB * 16];  // scratch of lds_trtri_blocked (ld kNB)
-   __shared__ int sh_bad;
-   typedef typename Mfma<T>::acc_t acc_t;
-   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-   const int m = nd.m, n = nd.n, ld = nd.ld;
-   for (int k0 = 0; k0 < n; k0 += kPB) {
-      const int kb = min(kPB, n - k0), kb16 = (kb + 15) & ~15;
-      T* blk = F + k0 + (int64_t)k0 * ld;
-      __syncthreads();  // the previous panel's update is complete
-      // diagonal block, padded to kb16 with the identity, upper triangle zero
-      for (int e = tid; e < kb16 * kb16; e += kThreads) {
-         const int i = e % kb16, j = e / kb16;
-         const bool live = i < kb && j < kb && i >= j;
-         const T v = *live_or_zero(live, blk + i + (int64_t)j * ld);
-         D[i + j * LD] = live ? v : ((i == j) ? T(1) : T(0));
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t col_window(T* F, int64_t ld, int col) {
+   return buf_rsrc(F + col * ld, 0xFFFFFFFFu);
+}
+
+// Accumulates NS 16-row strips of L(rows, 0:K) L(o:o+16, 0:K)^T: `ob` is the
+// lane's offset of the panel's own rows (strip 0 is those rows, so its two
+// operands are one load), oa[s] of the strips below. The loads of a chunk of
+// 4 KC columns are in flight while the chunk before it is multiplied (FP64:
+// as many as the registers of NS = 3 allow, 5 % on fronts of 384 rows and
+// more; FP32 no gain beyond 16 columns). K is a multiple of 16, cb the bytes
+// of a column; columns at or beyond K read zero.
+template <typename T, int NS>
+__device__ __forceinline__ void panel_products(T* F, int64_t ld, uint32_t cb, uint32_t ob, const uint32_t (&oa)[3],
+                                               int K, typename Mfma<T>::acc_t (&acc)[4]) {
+   constexpr int KC = sizeof(T) == 8 ? (NS == 1 ? 8 : NS == 2 ? 4 : 2) : 4;
+   T b[2][KC], a[2][KC][NS];
+   auto load = [&](int buf, int k) {
+      const auto rs = buf_rsrc(F + k * ld, (uint32_t)min(K - k, 4 * KC) * cb);
+#pragma unroll
+      for (int q = 0; q < KC; ++q) {
+         b[buf][q] = buf_load_s(rs, ob, 4 * q * cb, (T*)nullptr);
+#pragma unroll
+         for (int s = 0; s < NS; ++s) a[buf][q][s] = buf_load_s(rs, oa[s], 4 * q * cb, (T*)nullptr);
       }
-      __syncthreads();
-      const int bad = lds_potrf_panels<T, LD>(D, kb16, &sh_bad);
+   };
+   auto mul = [&](int buf, int k) {
+#pragma unroll
+      for (int q = 0; q < KC; ++q) {
+         if (q % 4 == 0 && k + 4 * q >= K) break;
+         acc[0] = Mfma<T>::op(b[buf][q], b[buf][q], acc[0]);
+#pragma unroll
+         for (int s = 0; s < NS; ++s) acc[s + 1] = Mfma<T>::op(b[buf][q], a[buf][q][s], acc[s + 1]);
+      }
+   };
+   if (K <= 0) return;
+   load(0, 0);
+   for (int k = 0;;) {
+      if (k + 4 * KC < K) load(1, k + 4 * KC);
+      mul(0, k);
+      k += 4 * KC;
+      if (k >= K) break;
+      if (k + 4 * KC < K) load(0, k + 4 * KC);
+      mul(1, k);
+      k += 4 * KC;
+      if (k >= K) break;
+   }
+}
+
+// Workgroup barrier for data exchanged through LDS: waits for the wave's LDS
+// operations only, its global stores stay in flight (__syncthreads would wait
+// for them).
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+template <typename T, int NT>
+__device__ __forceinline__ void front_potrf_block(const NodeDesc& nd, T* __restrict__ F, int* info_slot) {
+   constexpr int NW = NT / 64, LDB = 68;
+   constexpr uint32_t ES = sizeof(T);
+   // item v of an MFMA result lies in row/column rb(lane) + rstep v
+   constexpr int rstep = sizeof(T) == 8 ? 4 : 1;
+   __shared__ T tbuf[NW][16 * LDB];
+   __shared__ int sh_bad[2];  // by panel parity: written before, read after the panel's barrier
+   typedef typename Mfma<T>::acc_t acc_t;
+   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+   const int l16 = lane & 15, lq = lane >> 4, rb = Mfma<T>::row(lane, 0);
+   const int m = nd.m, n = nd.n;
+   const int64_t ld = nd.ld;
+   const uint32_t cb = (uint32_t)nd.ld * ES;
+   T* buf = tbuf[wave];
+   int ns_prev = 0;  // strips per wave of the panel before if its rows are all in tbuf, else 0
+   for (int o = 0; o < n; o += 16) {
+      const int kb = min(16, n - o);
+      const int below = m - o - kb;
+      // 16-row strips per wave and pass (the lanes hold 16 + 48 rows)
+      const int ns = min(3, ((below + 15) / 16 + NW - 1) / NW);
+      const bool one_pass = below <= NW * 16 * ns;
+      // the panel's columns: accesses beyond them read zero or are dropped
+      const auto pw = buf_rsrc(F + o * ld, kb * cb);
+      for (int w0 = o + kb + wave * 16 * ns, first = 1; first || w0 < m; w0 += NW * 16 * ns, first = 0) {
+         if (w0 >= m && wave != 0) {
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // its stores of the panel before, as below
+            if (one_pass) lds_barrier();
+            break;
+         }
+         // opaque copies: what is derived from them is formed where it is
+         // used instead of being kept (and spilled) over the panel loop
+         uint32_t cbp = cb;
+         int lp = lane;
+         asm volatile("" : "+s"(cbp), "+v"(lp));
+         const int row = lane < 16 ? o + lane : w0 + lane - 16;
+         const bool live = lane < 16 ? lane < kb : (row < m && lane < 16 + 16 * ns);
+         const uint32_t orow = live ? (uint32_t)row * ES : kOffMask;
+         T r[16];
+         acc_t acc[4] = {};
+         const uint32_t ob = (uint32_t)min(o + l16, m - 1) * ES + lq * cb;
+         uint32_t oa[3];
+#pragma unroll
+         for (int s = 0; s < 3; ++s) oa[s] = (uint32_t)min(w0 + s * 16 + l16, m - 1) * ES + lq * cb;
+         auto load_rows = [&] {
+#pragma unroll
+            for (int c = 0; c < 16; ++c) r[c] = buf_load_s(pw, orow, uniform(c * cbp), (T*)nullptr);
+         };
+         if (sizeof(T) == 4) load_rows();
+         const int K = ns_prev > 0 ? o - 16 : o;
+         if (ns <= 1)
+            panel_products<T, 1>(F, ld, cb, ob, oa, K, acc);
+         else if (ns == 2)
+            panel_products<T, 2>(F, ld, cb, ob, oa, K, acc);
+         else
+            panel_products<T, 3>(F, ld, cb, ob, oa, K, acc);
+         // FP64 loads them here, where the registers of the products are free
+         if (sizeof(T) == 8) load_rows();
+         if (ns_prev > 0) {
+            // the columns of the panel before, from the waves' buffers (wave w
+            // holds 16 ns_prev rows; the first 16 rows are this panel's own)
+            const T* bs = tbuf[0] + 16 + l16 + lq * LDB;
+            const T* as[3];
+#pragma unroll
+            for (int s = 0; s < 3; ++s) {
+               const int p = min(kb + 16 * (wave * ns + s) + l16, NW * 16 * ns_prev - 1);  // row in that panel
+               const int w = ns_prev == 1 ? p >> 4 : ns_prev == 2 ? p >> 5 : ((p >> 4) * 43) >> 7;
+               as[s] = tbuf[w] + 16 + p - 16 * ns_prev * w + lq * LDB;
+            }
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+               const T b = bs[4 * q * LDB];
+               acc[0] = Mfma<T>::op(b, b, acc[0]);
+#pragma unroll
+               for (int s = 0; s < 3; ++s)
+                  if (s < ns || s == 0) acc[s + 1] = Mfma<T>::op(b, as[s][4 * q * LDB], acc[s + 1]);
+            }
+         }
+         if (one_pass) {
+            // every wave has read the panel before and this diagonal block
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            lds_barrier();
+         }
+         // the products to a row per lane (item v of lane l is row l % 16,
+         // column row(l, v) of its strip), through the wave's own buffer
+#pragma unroll
+         for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) buf[(rb + rstep * v) * LDB + s * 16 + l16] = acc[s][v];
+         __builtin_amdgcn_wave_barrier();
+         T sum[16];
+#pragma unroll
+         for (int c = 0; c < 16; ++c) sum[c] = buf[c * LDB + lane];
+         // rows beyond the front and entries above the diagonal hold
+         // meaningless values: no other lane sees them
+#pragma unroll
+         for (int c = 0; c < 16; ++c) r[c] -= sum[c];
+         if (kb < 16) {
+            int kbp = kb;
+            asm volatile("" : "+s"(kbp));
+#pragma unroll
+            for (int c = 0; c < 16; ++c)
+               if (!live || c >= kbp) r[c] = T(lp == c ? 1 : 0);
+         }
+         __builtin_amdgcn_wave_barrier();
+         const int bad = panel_cholesky16(r, lane);
+         if (wave == 0 && lane == 0) sh_bad[(o >> 4) & 1] = bad;
+         // the stores of the panel before are complete (the next panel's
+         // products read them), this panel's stay in flight across its barrier.
+         // Wave 0 stores the diagonal block's lower triangle in the last pass.
+         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+         if (wave == 0) {
+            const int top = lane >= 16 ? 16 : (one_pass && live) ? lp : -1;  // last column stored
+#pragma unroll
+            for (int c = 0; c < 16; ++c) buf_store_s(pw, c <= top ? orow : kOffMask, uniform(c * cbp), r[c]);
+         } else {
+            const uint32_t os = lane >= 16 ? orow : kOffMask;
+#pragma unroll
+            for (int c = 0; c < 16; ++c) buf_store_s(pw, os, uniform(c * cbp), r[c]);
+         }
+#pragma unroll
+         for (int c = 0; c < 16; ++c) buf[c * LDB + lane] = r[c];
+      }
+      if (one_pass)
+         lds_barrier();
+      else
+         __syncthreads();
+      ns_prev = one_pass ? ns : 0;
+      const int bad = sh_bad[(o >> 4) & 1];
       if (bad) {
-         if (tid == 0) *info_slot = k0 + bad;
+         if (threadIdx.x == 0) *info_slot = o + bad;
          return;
       }
-      for (int e = tid; e < kb * kb; e += kThreads) {
-         const int i = e % kb, j = e / kb;
-         if (i >= j) blk[i + (int64_t)j * ld] = D[i + j * LD];
+      // several passes: the diagonal block (in wave 0's buffer since the last)
+      // once every wave has read its values; no later panel reads it
+      if (!one_pass && wave == 0) {
+         uint32_t cbp = cb;
+         int lp = lane < kb ? lane : -1;
+         asm volatile("" : "+s"(cbp), "+v"(lp));
+#pragma unroll
+         for (int c = 0; c < 16; ++c)
+            buf_store_s(pw, c <= lp ? (uint32_t)(o + lane) * ES : kOffMask, uniform(c * cbp), buf[c * LDB + lane]);
       }
-      __syncthreads();
-      lds_trtri_blocked<T, LD>(D, Tmp, kb16);  // D = inv(L11), lower
-      const int r0 = k0 + kb, R = m - r0;
-      if (R <= 0) continue;
-      // L21 = A21 inv(L11)^T in place. Operands: x = inv(L11)[c][k] (LDS),
-      // y = A21[row][k]; item v of lane l is L21[rs + l%16][16 ct + row(l, v)].
-      // All K operands of a strip or tile are loaded before its first product:
-      // one L2 round trip per tile instead of one per k-step.
-      constexpr int KS = kPB / 4;  // k-steps of a full panel
-      const int nct = kb16 / 16, nks = kb16 / 4;
-      for (int rs = r0 + wave * 16; rs < m; rs += 64) {
-         acc_t acc[kPB / 16];
+   }
+   __syncthreads();
+   // contribution block: C[i][j] -= sum_k L21[i][k] L21[j][k] over the lower
+   // triangle, a 32 x 32 tile (2 x 2 MFMA tiles) per wave; item v of lane l is
+   // C[i0 + l % 16][j0 + row(l, v)]
+   const int R = m - n;
+   const int nt = (R + 31) / 32;
+   const int ntiles = nt * (nt + 1) / 2;
+   constexpr int KC = sizeof(T) == 8 ? 2 : 4;
+   for (int tile = wave; tile < ntiles; tile += NW) {
+      int ti = (int)((__builtin_sqrtf(8.0f * tile + 1.0f) - 1.0f) * 0.5f);
+      while (ti * (ti + 1) / 2 > tile) --ti;
+      while ((ti + 1) * (ti + 2) / 2 <= tile) ++ti;
+      const int tj = tile - ti * (ti + 1) / 2;
+      const int ri = n + ti * 32, rj = n + tj * 32;
+      acc_t acc[2][2] = {};
+      uint32_t oi[2], oj[2];
 #pragma unroll
-         for (int ct = 0; ct < kPB / 16; ++ct) acc[ct] = acc_t{0, 0, 0, 0};
-         const int row = rs + (lane & 15);
-         T y[KS];
+      for (int u = 0; u < 2; ++u) {
+         oi[u] = (uint32_t)min(ri + u * 16 + l16, m - 1) * ES + lq * cb;
+         oj[u] = (uint32_t)min(rj + u * 16 + l16, m - 1) * ES + lq * cb;
+      }
+      T ya[2][KC][2], xb[2][KC][2];
+      auto load = [&](int bufi, int k) {
+         const auto rs = col_window(F, ld, k);
 #pragma unroll
-         for (int q = 0; q < KS; ++q) {
-            const int k = 4 * q + (lane >> 4);
-            y[q] = *live_or_zero(row < m && k < kb, F + row + (int64_t)(k0 + k) * ld);
+         for (int q = 0; q < KC; ++q) {
+            // columns beyond the pivots: zero
+            const uint32_t mask = k + 4 * q + lq < n ? 0u : kOffMask;
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+               ya[bufi][q][u] = buf_load_s(rs, oi[u] | mask, 4 * q * cb, (T*)nullptr);
+               xb[bufi][q][u] = buf_load_s(rs, oj[u] | mask, 4 * q * cb, (T*)nullptr);
+            }
          }
+      };
+      auto mul = [&](int bufi) {
 #pragma unroll
-         for (int q = 0; q < KS; ++q) {
-            if (q >= nks) break;
-            const int k = 4 * q + (lane >> 4);
+         for (int q = 0; q < KC; ++q)
 #pragma unroll
-            for (int ct = 0; ct < kPB / 16; ++ct)
-               if (ct < nct) acc[ct] = Mfma<T>::op(D[(ct * 16 + (lane & 15)) + k * LD], y[q], acc[ct]);
-         }
+            for (int x = 0; x < 2; ++x)
 #pragma unroll
-         for (int ct = 0; ct < kPB / 16; ++ct)
+               for (int y = 0; y < 2; ++y) acc[x][y] = Mfma<T>::op(xb[bufi][q][y], ya[bufi][q][x], acc[x][y]);
+      };
+      load(0, 0);
+      for (int k = 0;;) {
+         if (k + 4 * KC < n) load(1, k + 4 * KC);
+         mul(0);
+         k += 4 * KC;
+         if (k >= n) break;
+         if (k + 4 * KC < n) load(0, k + 4 * KC);
+         mul(1);
+         k += 4 * KC;
+         if (k >= n) break;
+      }
+      const auto cw = col_window(F, ld, rj);
+      T cv[2][2][4];
+      uint32_t oc[2][2][4];
+#pragma unroll
+      for (int x = 0; x < 2; ++x)
+#pragma unroll
+         for (int y = 0; y < 2; ++y)
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
-               const int c = ct * 16 + Mfma<T>::row(lane, v);
-               if (ct < nct && row < m && c < kb) F[row + (int64_t)(k0 + c) * ld] = acc[ct][v];
-            }
-      }
-      __syncthreads();  // L21 written before the update reads it
-      // trailing lower triangle: C[i][j] -= sum_k L21[i][k] L21[j][k] in
-      // 32 x 32 tiles (2 x 2 MFMA tiles per wave); operands x = L21[j][k],
-      // y = L21[i][k]; item v of lane l is C[i0 + l%16][j0 + row(l, v)].
-      const int nt = (R + 31) / 32;
-      const int ntiles = nt * (nt + 1) / 2;
-      for (int tile = wave; tile < ntiles; tile += 4) {
-         int ti = (int)((__builtin_sqrtf(8.0f * tile + 1.0f) - 1.0f) * 0.5f);
-         while (ti * (ti + 1) / 2 > tile) --ti;
-         while ((ti + 1) * (ti + 2) / 2 <= tile) ++ti;
-         const int tj = tile - ti * (ti + 1) / 2;
-         const int ri = r0 + ti * 32, rj = r0 + tj * 32;
-         acc_t acc[2][2];
-#pragma unroll
-         for (int a = 0; a < 2; ++a)
-#pragma unroll
-            for (int b = 0; b < 2; ++b) acc[a][b] = acc_t{0, 0, 0, 0};
-         // FP64: the operands in two halves of the panel (register budget)
-         constexpr int KC = sizeof(T) == 8 ? KS / 2 : KS;
-         for (int q0 = 0; q0 < nks; q0 += KC) {
-            T xa[2][KC], yb[2][KC];
-#pragma unroll
-            for (int q = 0; q < KC; ++q) {
-               const int k = 4 * (q0 + q) + (lane >> 4);
-#pragma unroll
-               for (int u = 0; u < 2; ++u) {
-                  const int i = ri + u * 16 + (lane & 15), j = rj + u * 16 + (lane & 15);
-                  yb[u][q] = *live_or_zero(i < m && k < kb, F + i + (int64_t)(k0 + k) * ld);
-                  xa[u][q] = *live_or_zero(j < m && k < kb, F + j + (int64_t)(k0 + k) * ld);
-               }
+               const int i = ri + x * 16 + l16, j = rj + y * 16 + rb + rstep * v;
+               oc[x][y][v] = (i < m && j <= i) ? (uint32_t)i * ES + rb * cb : kOffMask;
+               cv[x][y][v] = buf_load_s(cw, oc[x][y][v], (y * 16 + rstep * v) * cb, (T*)nullptr);
             }
 #pragma unroll
-            for (int q = 0; q < KC; ++q) {
-               if (q0 + q >= nks) break;
+      for (int x = 0; x < 2; ++x)
 #pragma unroll
-               for (int a = 0; a < 2; ++a)
+         for (int y = 0; y < 2; ++y)
 #pragma unroll
-                  for (int b = 0; b < 2; ++b) acc[a][b] = Mfma<T>::op(xa[b][q], yb[a][q], acc[a][b]);
-            }
-         }
-         T cv[2][2][4];
-#pragma unroll
-         for (int a = 0; a < 2; ++a)
-#pragma unroll
-            for (int b = 0; b < 2; ++b)
-#pragma unroll
-               for (int v = 0; v < 4; ++v) {
-                  const int i = ri + a * 16 + (lane & 15), j = rj + b * 16 + Mfma<T>::row(lane, v);
-                  cv[a][b][v] = *live_or_zero(i < m && j <= i, F + i + (int64_t)j * ld);
-               }
-#pragma unroll
-         for (int a = 0; a < 2; ++a)
-#pragma unroll
-            for (int b = 0; b < 2; ++b)
-#pragma unroll
-               for (int v = 0; v < 4; ++v) {
-                  const int i = ri + a * 16 + (lane & 15), j = rj + b * 16 + Mfma<T>::row(lane, v);
-                  if (i < m && j <= i) F[i + (int64_t)j * ld] = cv[a][b][v] - acc[a][b][v];
-               }
-      }
+            for (int v = 0; v < 4; ++v)
+               buf_store_s(cw, oc[x][y][v], (y * 16 + rstep * v) * cb, cv[x][y][v] - acc[x][y][v]);
    }
    __syncthreads();
 }
@@ -1351,17 +1559,18 @@ __global__ __launch_bounds__(kThreads) void k_small_asm(const int* __restrict__ 
       }
       ch = c.next_child;
    }
-   front_potrf_block<T>(nd, F, info + node);
+   __syncthreads();  // the front is assembled
+   front_potrf_block<T, kThreads>(nd, F, info + node);
 }
 
 template <typename T>
-__global__ __launch_bounds__(kThreads) void k_small_front(const int* __restrict__ node_list,
+__global__ __launch_bounds__(kFrontThreads, 4) void k_small_front(const int* __restrict__ node_list,
                                                           const NodeDesc* __restrict__ nodes,
                                                           T* __restrict__ arena,
                                                           int* __restrict__ info) {
    const int node = node_list[blockIdx.x];
    const NodeDesc nd = nodes[node];
-   front_potrf_block<T>(nd, arena + nd.off, info + node);
+   front_potrf_block<T, kFrontThreads>(nd, arena + nd.off, info + node);
 }
 
 // ---------------------------------------------------------------------------

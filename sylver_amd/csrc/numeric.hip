@@ -85,6 +85,31 @@ namespace {
 // the launch's width.
 constexpr int kStepMaxFronts = 64;
 
+// The fronts of `list` in decreasing order of their work (to a quarter of a
+// power of two, list order within a class): one-workgroup fronts are started
+// in launch order, so the largest no longer start last and run on alone.
+// m(f), n(f): rows and pivots of front f.
+template <typename M, typename N>
+void sort_by_work(int* list, size_t count, M&& m, N&& n) {
+   constexpr int kShift = 21;  // exponent and two bits of the mantissa
+   std::vector<uint32_t> key(count);
+   std::vector<int> start(1 << (32 - kShift), 0), in(list, list + count);
+   for (size_t i = 0; i < count; ++i) {
+      const float work = (float)node_flops(m(list[i]), n(list[i]));
+      uint32_t bits;
+      std::memcpy(&bits, &work, sizeof(bits));
+      key[i] = (uint32_t)start.size() - 1 - (bits >> kShift);
+      ++start[key[i]];
+   }
+   int at = 0;
+   for (int& b : start) {
+      const int c = b;
+      b = at;
+      at += c;
+   }
+   for (size_t i = 0; i < count; ++i) list[start[key[i]]++] = in[i];
+}
+
 // The plan's host side: layout, maps, task lists and launch programs. No
 // HIP call (it also runs, for its checks, on a host without a device).
 DevicePlan* build_plan_host(const Analysis& a, int small_max, int wide_ncol, int num_cus, const PlanKnobs& k) {
@@ -322,6 +347,8 @@ DevicePlan* build_plan_host(const Analysis& a, int small_max, int wide_ncol, int
          else
             large.push_back(i);
       }
+      sort_by_work(P->nlistv.data() + s0, P->nlistv.size() - s0, [&](int i) { return P->hnodes[i].m; },
+                   [&](int i) { return P->hnodes[i].n; });
       push(P->fprog, L_SMALL, s0, P->nlistv.size() - s0);
       // large fronts, block column by block column
       int maxn = 0;
@@ -1359,7 +1386,7 @@ void run_factor_program(const DevicePlan* P, DeviceFactors* F, hipStream_t s,
                                                              P->d_cmap, P->d_asmch, arena);
             break;
          case L_SMALL:
-            k_small_front<T><<<g, b, 0, s>>>(P->d_nlistv + L.off, P->d_nodes, arena, F->d_info);
+            k_small_front<T><<<g, dim3(kFrontThreads), 0, s>>>(P->d_nlistv + L.off, P->d_nodes, arena, F->d_info);
             break;
          case L_SMALL_ASM:
             k_small_asm<T><<<g, b, 0, s>>>(P->d_nlistv + L.off, P->d_nodes, P->d_nlist, P->d_rlist, F->d_aval,
@@ -2269,7 +2296,7 @@ double time_fronts_t(DevicePlan* P, DeviceFactors* F, const std::vector<int>& nr
    dfree(dl);
    dfree(doff);
    std::sort(t.begin(), t.end());
-   return t[t.size() / 2];
+   return t[(t.size() - 1) / 2];  // of an even count the lower one: an interrupted run only ever reads high
 }
 
 int time_fronts(int K, const int* m, const int* n, const signed char* variant, int precision, int reps,
@@ -2427,6 +2454,7 @@ int batched_front_potrf(int nfronts, const int* nrow, const int* ncol, const int
          nd[f].first_child = nd[f].next_child = -1;
          list[f] = f;
       }
+      sort_by_work(list.data(), list.size(), [&](int f) { return nrow[f]; }, [&](int f) { return ncol[f]; });
       hipStream_t s = static_cast<hipStream_t>(stream);
       NodeDesc* dnd = dalloc<NodeDesc>(nfronts);
       int* dl = dalloc<int>(nfronts);
@@ -2438,9 +2466,9 @@ int batched_front_potrf(int nfronts, const int* nrow, const int* ncol, const int
       HIPCHECK(hipEventCreate(&e1));
       HIPCHECK(hipEventRecord(e0, s));
       if (dtype == 0)
-         k_small_front<double><<<nfronts, kThreads, 0, s>>>(dl, dnd, static_cast<double*>(data), info);
+         k_small_front<double><<<nfronts, kFrontThreads, 0, s>>>(dl, dnd, static_cast<double*>(data), info);
       else
-         k_small_front<float><<<nfronts, kThreads, 0, s>>>(dl, dnd, static_cast<float*>(data), info);
+         k_small_front<float><<<nfronts, kFrontThreads, 0, s>>>(dl, dnd, static_cast<float*>(data), info);
       HIPCHECK(hipGetLastError());
       HIPCHECK(hipEventRecord(e1, s));
       HIPCHECK(hipStreamSynchronize(s));
@@ -2483,7 +2511,7 @@ static int64_t* scratch_ptr(int dev) {
 }
 
 template <typename T>
-__global__ __launch_bounds__(kThreads) void k_small_front_sized(const int64_t* __restrict__ off,
+__global__ __launch_bounds__(kFrontThreads, 4) void k_small_front_sized(const int64_t* __restrict__ off,
                                                                 const int* __restrict__ nrow,
                                                                 const int* __restrict__ ncol,
                                                                 T* __restrict__ data, int* __restrict__ info) {
@@ -2494,8 +2522,8 @@ __global__ __launch_bounds__(kThreads) void k_small_front_sized(const int64_t* _
    nd.ld = nd.m;
    nd.off = off[f];
    nd.first_child = nd.next_child = -1;
-   if (threadIdx.x == 0) info[f] = 0;  // front_potrf_block opens with a barrier
-   front_potrf_block<T>(nd, data + nd.off, info + f);
+   if (threadIdx.x == 0) info[f] = 0;  // the thread that reports a failing pivot
+   front_potrf_block<T, kFrontThreads>(nd, data + nd.off, info + f);
 }
 
 int batched_front_potrf_noalloc(int nfronts, const int* nrow, const int* ncol, const int64_t* off, void* data,
@@ -2519,10 +2547,10 @@ int batched_front_potrf_noalloc(int nfronts, const int* nrow, const int* ncol, c
       HIPCHECK(hipMemcpyAsync(s_nrow, nrow, nfronts * sizeof(int), hipMemcpyHostToDevice, s));
       HIPCHECK(hipMemcpyAsync(s_ncol, ncol, nfronts * sizeof(int), hipMemcpyHostToDevice, s));
       if (dtype == 0)
-         k_small_front_sized<double><<<nfronts, kThreads, 0, s>>>(s_off, s_nrow, s_ncol,
+         k_small_front_sized<double><<<nfronts, kFrontThreads, 0, s>>>(s_off, s_nrow, s_ncol,
                                                                    static_cast<double*>(data), info);
       else
-         k_small_front_sized<float><<<nfronts, kThreads, 0, s>>>(s_off, s_nrow, s_ncol,
+         k_small_front_sized<float><<<nfronts, kFrontThreads, 0, s>>>(s_off, s_nrow, s_ncol,
                                                                   static_cast<float*>(data), info);
       HIPCHECK(hipGetLastError());
       // the host arrays are the caller's and the scratch is shared: finish
