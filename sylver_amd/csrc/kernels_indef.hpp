@@ -27,6 +27,7 @@
 #include <cstdint>
 
 #include "kernels.hpp"
+#include "wave_ops.hpp"
 
 namespace sylver_amd {
 
@@ -87,48 +88,6 @@ __device__ inline void block_argmax(double& v, int& idx, double* sv, int* si) {
          idx = si[w];
       }
    __syncthreads();
-}
-
-// Two block-wide arg-max reductions at once (same rule as block_argmax);
-// `sv`/`si` hold 8 entries.
-__device__ inline void block_argmax2(double& v0, int& i0, double& v1, int& i1, double* sv, int* si) {
-#pragma unroll
-   for (int o = 32; o > 0; o >>= 1) {
-      const double a0 = __shfl_xor(v0, o), a1 = __shfl_xor(v1, o);
-      const int j0 = __shfl_xor(i0, o), j1 = __shfl_xor(i1, o);
-      if (a0 > v0 || (a0 == v0 && j0 < i0)) {
-         v0 = a0;
-         i0 = j0;
-      }
-      if (a1 > v1 || (a1 == v1 && j1 < i1)) {
-         v1 = a1;
-         i1 = j1;
-      }
-   }
-   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-   __syncthreads();
-   if (lane == 0) {
-      sv[wave] = v0;
-      si[wave] = i0;
-      sv[4 + wave] = v1;
-      si[4 + wave] = i1;
-   }
-   __syncthreads();
-   v0 = sv[0];
-   i0 = si[0];
-   v1 = sv[4];
-   i1 = si[4];
-#pragma unroll
-   for (int w = 1; w < kThreads / 64; ++w) {
-      if (sv[w] > v0 || (sv[w] == v0 && si[w] < i0)) {
-         v0 = sv[w];
-         i0 = si[w];
-      }
-      if (sv[4 + w] > v1 || (sv[4 + w] == v1 && si[4 + w] < i1)) {
-         v1 = sv[4 + w];
-         i1 = si[4 + w];
-      }
-   }
 }
 
 __device__ inline double block_max(double v, double* sv) {
@@ -243,110 +202,181 @@ __device__ __forceinline__ double vs_value(const double* dl, int p, int npass, d
 // Bunch-Parlett LDL^T of the kb x kb diagonal block T (LDS, both triangles
 // on entry) with complete pivoting inside the block (alpha = (1 + sqrt 17) / 8):
 // 1x1 pivots [d^{-1}, 0] and 2x2 pivots [a, b, inf, c] into dl, L below the
-// diagonal of T. `swap_local(p, q)` exchanges positions p and q of the block
-// (T and whatever the caller keeps in step). A pivot below `small` ends the
+// diagonal of T (what is above it is meaningless afterwards), and into perm
+// the row of the block at each position. A pivot below `small` ends the
 // block: with action the rest is zero pivots, without it the return is 1.
-// All threads call; the result is uniform.
-template <typename Swap>
-__device__ int bp_block(double (*T)[kAppNB + 1], double* dl, int kb, double small, int action,
-                        double* red_v, int* red_i, Swap&& swap_local) {
+// All kThreads threads call; the result is uniform.
+//
+// The trailing block is held in registers, full and symmetric: lane r of
+// wave w holds row r, columns w, w + 4, ... Rows and columns keep their
+// places; `pos` is a row's position under the exchanges so far, and decides
+// which of the two operands of an entry's update is L (the row in the later
+// position) and which entry of equal ones is the pivot (the first by column,
+// then row). A step costs the wave a scan of its 16 entries per lane, a DPP
+// maximum, two barriers (maxima; the pivot's row, written by the lanes that
+// hold it) and 16 updates: about a thousand cycles. In LDS, with the
+// exchanges done, a 64-column block took 247 us.
+constexpr double kBpAlpha = 0.6403882032022076;
+
+struct BpScratch {
+   double mx[4];       // per wave: largest entry
+   int key[4];         // per wave: position key of the first entry equal to the largest
+   double col[2][64];  // the pivot rows
+};
+
+__device__ __forceinline__ int bp_block(double (*T)[kAppNB + 1], double* dl, int* perm, int kb, double small, int action,
+                                        BpScratch& sc) {
 #pragma clang fp contract(off)
-   // thread (ti, tj): row s + ti (or s + 1 + ti ...) of the trailing block,
-   // columns tj, tj + 4, ... of it
-   const int tid = threadIdx.x, ti = tid & 63, tj = tid >> 6;
-   for (int s = 0; s < kb;) {
-      double v0 = -1.0, v1 = -1.0;
-      int i0 = 0x7fffffff, i1 = 0x7fffffff;
-      {
-         const int i = s + ti;
-         if (i < kb)
-            for (int j = s + tj; j <= i; j += 4) {
-               const double v = fabs(T[i][j]);
-               const int idx = j * kb + i;
-               if (v > v0 || (v == v0 && idx < i0)) {
-                  v0 = v;
-                  i0 = idx;
-               }
-               if (i == j && (v > v1 || (v == v1 && i < i1))) {
-                  v1 = v;
-                  i1 = i;
-               }
-            }
-      }
-      block_argmax2(v0, i0, v1, i1, red_v, red_i);
+   static_assert(kAppNB == 64 && kThreads == 256, "a row per lane, 16 columns per wave");
+   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+   auto dmax = [](double p, double q) { return q > p ? q : p; };
+   auto imin = [](int p, int q) { return min(p, q); };
+   int pos = lane < kb ? lane : -1;
+   double t[16], dg = lane < kb ? T[lane][lane] : 0.0;
+   unsigned act = 0;  // active columns of the wave
+#pragma unroll
+   for (int u = 0; u < 16; ++u) {
+      const int c = 4 * u + wave;
+      t[u] = (lane < kb && c < kb) ? T[lane][c] : 0.0;
+      act |= (c < kb ? 1u : 0u) << u;
+   }
+   __syncthreads();  // T is overwritten with L from here on
+   auto row_at = [&](int position) {
+      const unsigned long long b = __ballot(pos == position);
+      return b ? (int)__builtin_ctzll(b) : 0;
+   };
+   // the rows at position s and at lane p change places
+   auto to_front = [&](int s, int p) {
+      const int was = lane_value(pos, p);
+      pos = lane == p ? s : pos == s ? was : pos;
+      if ((p & 3) == wave) act &= ~(1u << (p >> 2));
+   };
+   int bad = 0, s = 0;
+   while (s < kb) {
+      double v = -1.0;
+#pragma unroll
+      for (int u = 0; u < 16; ++u)
+         if (act >> u & 1) v = dmax(v, fabs(t[u]));
+      v = wave_reduce(pos >= s ? v : -1.0, dmax);
+      if (lane == 0) sc.mx[wave] = v;
+      // largest diagonal entry, the smallest position among equal ones (every wave for itself)
+      const double ad = pos >= s ? dmax(-1.0, fabs(dg)) : -1.0;
+      const double v1 = wave_reduce(ad, dmax);
+      const unsigned long long hit = __ballot(pos >= s && ad == v1);
+      int p = __builtin_popcountll(hit) == 1
+                  ? (int)__builtin_ctzll(hit)
+                  : row_at(wave_reduce(pos >= s && ad == v1 ? pos : 0x7fffffff, imin));
+      __syncthreads();
+      const double v0 = dmax(dmax(sc.mx[0], sc.mx[1]), dmax(sc.mx[2], sc.mx[3]));
       if (v0 < small) {
-         if (!action) return 1;
-         for (int k = s + tid; k < kb; k += kThreads) {
-            dl[2 * k] = 0.0;
-            dl[2 * k + 1] = 0.0;
+         if (!action) {
+            bad = 1;
+            break;
          }
-         {
-            const int i = s + ti;
-            if (i < kb)
-               for (int j = s + tj; j < i; j += 4) T[i][j] = 0.0;
+         if (wave == 0) {
+            if (pos >= s) {
+               dl[2 * pos] = 0.0;
+               dl[2 * pos + 1] = 0.0;
+               for (int j = s; j < kb; ++j) T[lane][j] = 0.0;
+            }
          }
-         __syncthreads();
          break;
       }
-      // the trailing update also writes the mirror entry, so that the
-      // trailing block stays symmetric for the next exchanges
-      if (v1 >= 0.6403882032022076 * v0) {
-         swap_local(s, i1);
-         const double dv = T[s][s];
-         const double d0 = 1.0 / dv;
-         if (tid == 0) {
-            dl[2 * s] = d0;
-            dl[2 * s + 1] = 0.0;
-         }
-         {
-            const int i = s + 1 + ti;
-            if (i < kb)
-               for (int j = s + 1 + tj; j <= i; j += 4) {
-                  const double li = T[i][s] * d0;
-                  const double x = fnma(li, T[j][s], T[i][j]);
-                  T[i][j] = x;
-                  if (j < i) T[j][i] = x;
-               }
-         }
+      if (v1 >= kBpAlpha * v0) {
+         const double d0 = 1.0 / lane_value(dg, p);
+         to_front(s, p);
+         if (lane == p)
+#pragma unroll
+            for (int u = 0; u < 16; ++u) sc.col[0][4 * u + wave] = t[u];
          __syncthreads();
-         for (int i = s + 1 + tid; i < kb; i += kThreads) T[i][s] = T[i][s] * d0;
+         const double br = sc.col[0][lane], lr = br * d0;
+         if (wave == 0) {
+            if (pos > s) T[lane][s] = lr;
+            if (lane == 0) {
+               dl[2 * s] = d0;
+               dl[2 * s + 1] = 0.0;
+            }
+         }
+         dg = fnma(lr, br, dg);
+#pragma unroll
+         for (int u = 0; u < 16; ++u)
+            if (act >> u & 1) {
+               const double bc = lane_value(t[u], p), lc = bc * d0;
+               const bool low = pos >= lane_value(pos, 4 * u + wave);
+               t[u] = fnma(low ? lr : lc, low ? bc : br, t[u]);
+            }
          s += 1;
       } else {
-         int j0 = i0 / kb, ii0 = i0 % kb;
-         swap_local(s, j0);
-         if (ii0 == s) ii0 = j0;
-         swap_local(s + 1, ii0);
-         const double a = T[s][s], b = T[s + 1][s], c = T[s + 1][s + 1];
+         // the largest entry, off the diagonal: the first by (column, row) position
+         int key = 0x7fffffff;
+#pragma unroll
+         for (int u = 0; u < 16; ++u)
+            if (act >> u & 1) {
+               const int pc = lane_value(pos, 4 * u + wave);
+               const int k = min(pos, pc) * kb + max(pos, pc);
+               if (pos >= s && fabs(t[u]) == v0) key = min(key, k);
+            }
+         key = wave_reduce(key, imin);
+         if (lane == 0) sc.key[wave] = key;
+         __syncthreads();
+         key = min(min(sc.key[0], sc.key[1]), min(sc.key[2], sc.key[3]));
+         key = __builtin_amdgcn_readfirstlane(key);
+         const int j0 = key / kb;
+         int i0 = key - j0 * kb;
+         p = row_at(j0);
+         to_front(s, p);
+         if (i0 == s) i0 = j0;
+         const int q = row_at(i0);
+         to_front(s + 1, q);
+         if (lane == p)
+#pragma unroll
+            for (int u = 0; u < 16; ++u) sc.col[0][4 * u + wave] = t[u];
+         if (lane == q)
+#pragma unroll
+            for (int u = 0; u < 16; ++u) sc.col[1][4 * u + wave] = t[u];
+         const double a = lane_value(dg, p), c = lane_value(dg, q);
+         __syncthreads();
+         const double b = sc.col[0][q];
          const double det = __builtin_fma(a, c, -(b * b));
          const double d0 = c / det, d1 = -b / det, d3 = a / det;
-         if (tid == 0) {
-            dl[2 * s] = d0;
-            dl[2 * s + 1] = d1;
-            dl[2 * s + 2] = __builtin_inf();
-            dl[2 * s + 3] = d3;
+         const double r1 = sc.col[0][lane], r2 = sc.col[1][lane];
+         const double l0 = dot2(d0, r1, d1, r2), l1 = dot2(d1, r1, d3, r2);
+         if (wave == 0) {
+            if (pos > s + 1) {
+               T[lane][s] = l0;
+               T[lane][s + 1] = l1;
+            }
+            if (lane == 0) {
+               T[q][s] = 0.0;
+               dl[2 * s] = d0;
+               dl[2 * s + 1] = d1;
+               dl[2 * s + 2] = __builtin_inf();
+               dl[2 * s + 3] = d3;
+            }
          }
-         {
-            const int i = s + 2 + ti;
-            if (i < kb)
-               for (int j = s + 2 + tj; j <= i; j += 4) {
-                  const double a1 = T[i][s], a2 = T[i][s + 1];
-                  const double l0 = dot2(d0, a1, d1, a2), l1 = dot2(d1, a1, d3, a2);
-                  const double x = fnma(l1, T[j][s + 1], fnma(l0, T[j][s], T[i][j]));
-                  T[i][j] = x;
-                  if (j < i) T[j][i] = x;
-               }
-         }
-         __syncthreads();
-         for (int i = s + 2 + tid; i < kb; i += kThreads) {
-            const double a1 = T[i][s], a2 = T[i][s + 1];
-            T[i][s] = dot2(d0, a1, d1, a2);
-            T[i][s + 1] = dot2(d1, a1, d3, a2);
-         }
-         if (tid == 0) T[s + 1][s] = 0.0;
+         dg = fnma(l1, r2, fnma(l0, r1, dg));
+#pragma unroll
+         for (int u = 0; u < 16; ++u)
+            if (act >> u & 1) {
+               const double c1 = lane_value(t[u], p), c2 = lane_value(t[u], q);
+               const double k0 = dot2(d0, c1, d1, c2), k1 = dot2(d1, c1, d3, c2);
+               const bool low = pos >= lane_value(pos, 4 * u + wave);
+               t[u] = fnma(low ? l1 : k1, low ? c2 : r2, fnma(low ? l0 : k0, low ? c1 : r1, t[u]));
+            }
          s += 2;
       }
-      __syncthreads();
    }
+   __syncthreads();
+   if (bad) return 1;
+   // the rows of L to their positions
+#pragma unroll
+   for (int u = 0; u < 16; ++u) t[u] = T[lane][4 * u + wave];
+   if (wave == 0 && pos >= 0) perm[pos] = lane;
+   __syncthreads();
+#pragma unroll
+   for (int u = 0; u < 16; ++u)
+      if (4 * u + wave < pos) T[pos][4 * u + wave] = t[u];
+   __syncthreads();
    return 0;
 }
 
@@ -518,8 +548,10 @@ static __global__ __launch_bounds__(kThreads) void k_app_front(const int* __rest
    __shared__ double T[NB][NB + 1];
    __shared__ double VS[NB][NB + 1];
    __shared__ double dl[2 * NB];
+   __shared__ BpScratch sc;
    __shared__ double red_v[8];
    __shared__ int red_i[8];
+   __shared__ int perm[NB];
    __shared__ int s_fail, s_npass, s_bad;
    const int node = list[blockIdx.x];
    const IndefDesc nd = nodes[node];
@@ -554,48 +586,60 @@ static __global__ __launch_bounds__(kThreads) void k_app_front(const int* __rest
    int nelim = 0;
    for (int c0 = 0; c0 < n; c0 += NB) {
       const int kb = min(NB, n - c0);
-      for (int64_t e = tid; e < (int64_t)kb * m; e += kThreads) {
-         const int i = (int)(e % m), j = (int)(e / m);
-         Bk[i + (int64_t)j * m] = F[i + (int64_t)(c0 + j) * ld];
-      }
-      for (int e = tid; e < kb * kb; e += kThreads) {
-         const int i = e % kb, j = e / kb;
-         T[i][j] = F[c0 + i + (int64_t)(c0 + j) * ld];
+      for (int e = tid; e < NB * NB; e += kThreads) {
+         const int i = e & (NB - 1), j = e / NB;
+         if (i < kb && j < kb) VS[i][j] = T[i][j] = F[c0 + i + (int64_t)(c0 + j) * ld];
       }
       __syncthreads();
       // ---- Bunch-Parlett LDL^T of the diagonal block (in LDS) ----
-      auto swap_local = [&](int p, int q) {
-         if (p == q) return;
-         for (int k = tid; k < kb; k += kThreads) {
-            double a = T[k][p];
-            T[k][p] = T[k][q];
-            T[k][q] = a;
-         }
-         __syncthreads();
-         for (int k = tid; k < kb; k += kThreads) {
-            double a = T[p][k];
-            T[p][k] = T[q][k];
-            T[q][k] = a;
-         }
-         for (int k = tid; k < m; k += kThreads) {
-            double a = Bk[k + (int64_t)p * m];
-            Bk[k + (int64_t)p * m] = Bk[k + (int64_t)q * m];
-            Bk[k + (int64_t)q * m] = a;
-         }
-         __syncthreads();
-         for (int k = tid; k < kb; k += kThreads) {
-            double a = Bk[c0 + p + (int64_t)k * m];
-            Bk[c0 + p + (int64_t)k * m] = Bk[c0 + q + (int64_t)k * m];
-            Bk[c0 + q + (int64_t)k * m] = a;
-         }
-         __syncthreads();
-         front_swap(F, ld, m, n, c0 + p, c0 + q, var, pre);
-      };
-      if (bp_block(T, dl, kb, small, action, red_v, red_i, swap_local)) {
+      if (bp_block(T, dl, perm, kb, small, action, sc)) {
          if (tid == 0) s_bad = 1;
-         __syncthreads();
+         break;
       }
-      if (s_bad) break;
+      // the exchanges of the block in one pass: its columns over all rows
+      // (backed up as they are now), its rows over the fully-summed columns
+      for (int r = tid; r < m; r += kThreads) {
+         if (r >= c0 && r < c0 + kb) continue;
+         double x[NB];
+#pragma unroll
+         for (int j = 0; j < NB; ++j) x[j] = (j < kb) ? F[r + (int64_t)(c0 + perm[j]) * ld] : 0.0;
+#pragma unroll
+         for (int j = 0; j < NB; ++j)
+            if (j < kb) {
+               F[r + (int64_t)(c0 + j) * ld] = x[j];
+               Bk[r + (int64_t)j * m] = x[j];
+            }
+      }
+      for (int k = tid; k < n; k += kThreads) {
+         if (k >= c0 && k < c0 + kb) continue;
+         double x[NB];
+#pragma unroll
+         for (int j = 0; j < NB; ++j) x[j] = (j < kb) ? F[c0 + perm[j] + (int64_t)k * ld] : 0.0;
+#pragma unroll
+         for (int j = 0; j < NB; ++j)
+            if (j < kb) F[c0 + j + (int64_t)k * ld] = x[j];
+      }
+      {
+         int vv = 0, pp = 0;
+         if (tid < kb) {
+            vv = var[c0 + perm[tid]];
+            pp = pre[c0 + perm[tid]];
+         }
+         __syncthreads();
+         for (int e = tid; e < NB * NB; e += kThreads) {
+            const int i = e & (NB - 1), j = e / NB;
+            if (i < kb && j < kb) {
+               const double x = VS[perm[i]][perm[j]];
+               F[c0 + i + (int64_t)(c0 + j) * ld] = x;
+               Bk[c0 + i + (int64_t)j * m] = x;
+            }
+         }
+         if (tid < kb) {
+            var[c0 + tid] = vv;
+            pre[c0 + tid] = pp;
+         }
+      }
+      __syncthreads();
       // ---- ApplyN / ApplyT on every other uneliminated row + threshold ----
       if (tid == 0) s_fail = kb;
       __syncthreads();
@@ -640,10 +684,10 @@ static __global__ __launch_bounds__(kThreads) void k_app_front(const int* __rest
       // ---- update of the uneliminated fully-summed columns ----
       if (npass > 0) {
          for (int s0 = 0; s0 < n; s0 += NB) {
-            const int sc = min(NB, n - s0);
+            const int sc_n = min(NB, n - s0);
             // VS[t][p] = (D L[s, :])_p for column s = s0 + t
-            for (int e = tid; e < sc * npass; e += kThreads) {
-               const int t = e % sc, p = e / sc;
+            for (int e = tid; e < sc_n * npass; e += kThreads) {
+               const int t = e % sc_n, p = e / sc_n;
                const int s = s0 + t;
                const double* fs = F + s + (int64_t)c0 * ld;
                const double fm = p > 0 ? fs[(int64_t)(p - 1) * ld] : 0.0;
@@ -651,28 +695,37 @@ static __global__ __launch_bounds__(kThreads) void k_app_front(const int* __rest
                VS[t][p] = vs_value(dl, p, npass, fm, fs[(int64_t)p * ld], fp);
             }
             __syncthreads();
-            for (int r = tid; r < m; r += kThreads) {
-               if (EL[r] || (r >= c0 && r < c0 + npass)) continue;
+            // the lower triangle, four columns at a time (four independent
+            // chains of sums); the fully-summed part mirrored as it is written
+            for (int r = s0 / kThreads * kThreads + tid; r < m; r += kThreads) {
+               if (r < s0 || EL[r] || (r >= c0 && r < c0 + npass)) continue;
                double lr[NB];
 #pragma unroll
                for (int p = 0; p < NB; ++p) lr[p] = (p < npass) ? F[r + (int64_t)(c0 + p) * ld] : 0.0;
-               for (int t = 0; t < sc; ++t) {
-                  const int s = s0 + t;
-                  if (EL[s] || (s >= c0 && s < c0 + npass)) continue;
-                  double x = F[r + (int64_t)s * ld];
+               for (int t = 0; t < sc_n && s0 + t <= r; t += 4) {
+                  double x[4];
+                  bool live[4];
+#pragma unroll
+                  for (int k = 0; k < 4; ++k) {
+                     const int s = s0 + t + k;
+                     live[k] = t + k < sc_n && s <= r && !EL[min(s, n - 1)] && !(s >= c0 && s < c0 + npass);
+                     x[k] = live[k] ? F[r + (int64_t)s * ld] : 0.0;
+                  }
 #pragma unroll
                   for (int p = 0; p < NB; ++p)
-                     if (p < npass) x = fnma(lr[p], VS[t][p], x);
-                  F[r + (int64_t)s * ld] = x;
+                     if (p < npass)
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) x[k] = fnma(lr[p], VS[t + k][p], x[k]);
+#pragma unroll
+                  for (int k = 0; k < 4; ++k) {
+                     const int s = s0 + t + k;
+                     if (!live[k]) continue;
+                     F[r + (int64_t)s * ld] = x[k];
+                     if (r < n && r != s) F[s + (int64_t)r * ld] = x[k];
+                  }
                }
             }
             __syncthreads();
-         }
-         // symmetric copy of the updated fully-summed block
-         for (int64_t e = tid; e < (int64_t)n * n; e += kThreads) {
-            const int i = (int)(e % n), j = (int)(e / n);
-            if (i > j && !EL[i] && !EL[j] && !(i >= c0 && i < c0 + npass) && !(j >= c0 && j < c0 + npass))
-               F[j + (int64_t)i * ld] = F[i + (int64_t)j * ld];
          }
       }
       __syncthreads();
@@ -684,6 +737,7 @@ static __global__ __launch_bounds__(kThreads) void k_app_front(const int* __rest
       nelim += npass;
       __syncthreads();
    }
+   __syncthreads();
    if (s_bad) {
       if (tid == 0) {
          status[node] = -5;
@@ -861,8 +915,7 @@ static __global__ __launch_bounds__(kThreads) void k_lp_diag(int node, int c0, i
    constexpr int NB = kAppNB;
    __shared__ double T[NB][NB + 1];
    __shared__ double dl[2 * NB];
-   __shared__ double red_v[8];
-   __shared__ int red_i[8];
+   __shared__ BpScratch sc;
    __shared__ int perm[NB];
    const IndefDesc nd = nodes[node];
    const int m = nd.m, n = nd.n, ld = nd.ld, tid = threadIdx.x;
@@ -874,29 +927,8 @@ static __global__ __launch_bounds__(kThreads) void k_lp_diag(int node, int c0, i
       const int i = e % kb, j = e / kb;
       T[i][j] = F[c0 + i + (int64_t)(c0 + j) * ld];
    }
-   if (tid < NB) perm[tid] = tid;
    __syncthreads();
-   auto swap_local = [&](int p, int q) {
-      if (p == q) return;
-      for (int k = tid; k < kb; k += kThreads) {
-         const double a = T[k][p];
-         T[k][p] = T[k][q];
-         T[k][q] = a;
-      }
-      __syncthreads();
-      for (int k = tid; k < kb; k += kThreads) {
-         const double a = T[p][k];
-         T[p][k] = T[q][k];
-         T[q][k] = a;
-      }
-      if (tid == 0) {
-         const int t = perm[p];
-         perm[p] = perm[q];
-         perm[q] = t;
-      }
-      __syncthreads();
-   };
-   if (bp_block(T, dl, kb, small, action, red_v, red_i, swap_local)) {
+   if (bp_block(T, dl, perm, kb, small, action, sc)) {
       if (tid == 0) w.ST[kStBad] = 1;
       return;
    }

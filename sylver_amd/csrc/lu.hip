@@ -28,6 +28,7 @@
 #include <vector>
 
 #include "numeric.hpp"
+#include "wave_ops.hpp"
 
 namespace sylver_amd {
 
@@ -45,46 +46,6 @@ struct LuTask {
 template <typename T>
 __device__ inline T lu_abs(T v) {
    return v < T(0) ? -v : v;
-}
-
-// v from another lane by a DPP control; lanes without a source keep v.
-template <int CTRL>
-__device__ __forceinline__ int dpp(int v) {
-   return __builtin_amdgcn_update_dpp(v, v, CTRL, 0xf, 0xf, false);
-}
-template <int CTRL>
-__device__ __forceinline__ float dpp(float v) {
-   return __int_as_float(dpp<CTRL>(__float_as_int(v)));
-}
-template <int CTRL>
-__device__ __forceinline__ double dpp(double v) {
-   const long long u = __double_as_longlong(v);
-   const int lo = dpp<CTRL>((int)(u & 0xffffffff)), hi = dpp<CTRL>((int)(u >> 32));
-   return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-}
-
-__device__ __forceinline__ int lane_value(int v, int lane) { return __builtin_amdgcn_readlane(v, lane); }
-__device__ __forceinline__ float lane_value(float v, int lane) {
-   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
-}
-__device__ __forceinline__ double lane_value(double v, int lane) {
-   const long long u = __double_as_longlong(v);
-   const int lo = __builtin_amdgcn_readlane((int)(u & 0xffffffff), lane);
-   const int hi = __builtin_amdgcn_readlane((int)(u >> 32), lane);
-   return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-}
-
-// Reduction over the wave by `op` (associative, idempotent): row scans, then
-// the rows' last lanes onward; lane 63 ends with the result.
-template <typename V, typename Op>
-__device__ __forceinline__ V wave_reduce(V v, Op op) {
-   v = op(v, dpp<0x111>(v));  // row_shr:1
-   v = op(v, dpp<0x112>(v));
-   v = op(v, dpp<0x114>(v));
-   v = op(v, dpp<0x118>(v));
-   v = op(v, dpp<0x142>(v));  // row_bcast:15
-   v = op(v, dpp<0x143>(v));  // row_bcast:31
-   return lane_value(v, 63);
 }
 
 // The columns of a wave, one register (pair) per column and row set: vectors,
