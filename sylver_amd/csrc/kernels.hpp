@@ -1714,6 +1714,9 @@ __device__ __forceinline__ void solve_step_dev(const SolveTask& t, const NodeDes
          av[u] = *live_or_zero(ui < t.r1 && k < kb, p);
       }
    }
+   // rows of y beyond a short block meet zero columns of L in the products
+   // below: they must not hold whatever the LDS held before
+   for (int e = (kb & ~15) * 16 + threadIdx.x; e < kNB * 16; e += kThreads) ys[e] = 0.0;
    for (int c0 = 0; c0 < nrhs; c0 += 16) {
       const int nc = min(16, nrhs - c0);
       __syncthreads();
