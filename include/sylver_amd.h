@@ -163,7 +163,8 @@ typedef struct {
    int small_front_max;  /* fronts with nrow <= this use the one-workgroup kernel (0 = auto) */
    int record_timing;    /* record per-level device timings (0) */
    int indef_panel_min;  /* indefinite fronts with at least this many fully-summed columns
-                            use the multi-workgroup APP panel (0 = auto: 256) */
+                            use the multi-workgroup APP panel (0 = auto: 80, or fewer on
+                            fronts of many rows) */
    int small_assembly;   /* one-workgroup posdef fronts: 1 assembled (zero, A entries,
                             children) inside their factor launch, one launch per level;
                             0 separate zero / scatter / extend-add launches (default:

@@ -162,9 +162,9 @@ void large_panel(IndefState& S, int node, int slot, double u, double small, int 
       const int kb = std::min(kAppNB, n - c0), par = k & 1;
       const bool next = c0 + kb < n;
       if (k > 0) HIPCHECK(hipStreamWaitEvent(s, S.ev[1], 0));
-      k_lp_perm<<<1 + grid_cap((int64_t)m + n, 1024), kThreads, 0, s>>>(node, c0, S.d_nodes, S.arena, S.d_vars,
+      k_lp_perm<<<1 + grid_cap(64 * ((int64_t)(m + 63) / 64 + n), 1024), kThreads, 0, s>>>(node, c0, S.d_nodes, S.arena, S.d_vars,
                                                                        S.d_pres, S.d_ws);
-      k_lp_apply<<<grid_cap((int64_t)m - kb, 1024), kThreads, 0, s>>>(node, c0, par, S.d_nodes, S.arena, S.d_ws,
+      k_lp_apply<<<grid_cap(((int64_t)m - kb) * (kThreads / 64), 4096), 64, 0, s>>>(node, c0, par, S.d_nodes, S.arena, S.d_ws,
                                                                        u, small);
       k_lp_finish<<<1, kThreads, 0, s>>>(node, c0, par, S.d_nodes, S.arena, S.d_dinv, S.d_ws);
       HIPCHECK(hipEventRecord(S.ev[0], s));
@@ -267,12 +267,18 @@ void factor_indef(const Analysis& a, const DevicePlan* P, DeviceFactors* F, cons
    // FP32, FP64 fronts); pivot tests, D and its inverse stay FP64
    const bool low = F->precision != SYLVER_AMD_PREC_FP64;
    // fronts on the multi-workgroup panel: at least panel_min fully-summed
-   // columns; in auto mode also fronts of 2^18 entries or more (many
-   // rows, where one workgroup's pass over all rows per pivot is slow)
+   // columns; in auto mode 80, or 48 K entries (many rows, where one
+   // workgroup's pass over all rows per second-pass pivot is slow). Its
+   // launches of one front follow one another, while the one-workgroup fronts
+   // of a level run side by side: below the line the level's slowest front
+   // costs less than the sum of its panels. KKT factorizations with 256
+   // columns / 256 K entries, 64 / 256 K, 80 / 48 K (grid 8^3 + 128 rows 3.7,
+   // 2.9, 2.9 ms; 16^3 + 1024 54.9, 32.2, 31.8; 20^3 + 2000 87.1, 74.7, 73.2;
+   // 24^3 + 3456 151, 136.7, 135.7); from 32 K entries on the last gets slower
    const int panel_opt = ext_options().indef_panel_min;
-   const int panel_min = panel_opt > 0 ? panel_opt : 256;
+   const int panel_min = panel_opt > 0 ? panel_opt : 80;
    auto is_large = [&](const IndefDesc& d) {
-      return d.n >= panel_min || (panel_opt <= 0 && (int64_t)d.m * d.n >= (int64_t(1) << 18));
+      return d.n >= panel_min || (panel_opt <= 0 && (int64_t)d.m * d.n >= 3 * (int64_t(1) << 14));
    };
    const int failed_tpp = (opts.failed_pivot_method == 1 || opts.pivot_method == 3) ? 1 : 0;
    int64_t vars_used = 0, pres_used = 0, dinv_used = 0, x_used = 0, lf_used = 0, cb_used = 0;

@@ -142,27 +142,60 @@ __device__ __forceinline__ void apply_dinv1(double d0, double small, double& x) 
 // src/kernels/ldlt_app.hxx:144-255): x holds the row's kb entries in the
 // block columns; x := x L11^{-T} D^{-1} with the unit lower L11 of T and the
 // D^{-1} entries dl. Returns the first column with |l| > 1/u (kb if none).
-__device__ __forceinline__ int apply_row(double (&x)[kAppNB], const double (*T)[kAppNB + 1],
-                                         const double* dl, int kb, double small, double inv_u) {
+// Tt is L11 transposed: entry (j, i) at Tt[i][j], zero from row kb on (where
+// x is zero as well). Row i of Tt at a time, so that the products of a step
+// are independent -- each entry still receives its own in the order i = 0, 1,
+// ... -- and in chunks of 16 entries, the next chunk read from LDS while one
+// is multiplied (left to itself the compiler waits for every read: 62 us for
+// a block of 3300 rows).
+constexpr int kTtLd = kAppNB + 2;  // rows of 16-byte aligned pairs
+
+template <int B>  // rows 16 B .. 16 B + 15 of Tt
+__device__ __forceinline__ void apply_rows16(double (&x)[kAppNB], const double (*Tt)[kTtLd]) {
 #pragma clang fp contract(off)
+   typedef double d2 __attribute__((ext_vector_type(2)));
+   constexpr int NC = kAppNB / 16 - B;  // chunks of a row: columns 16 B .. 63
+   d2 t[2][8];
+   auto load = [&](int q) {
 #pragma unroll
-   for (int j = 1; j < kAppNB; ++j)
+      for (int e = 0; e < 8; ++e)
+         t[q & 1][e] = *reinterpret_cast<const d2*>(&Tt[16 * B + q / NC][16 * (B + q % NC) + 2 * e]);
+   };
+   load(0);
 #pragma unroll
-      for (int i = 0; i < j; ++i)
-         if (j < kb) x[j] = fnma(x[i], T[j][i], x[j]);
+   for (int q = 0; q < 16 * NC; ++q) {
+      if (q + 1 < 16 * NC) load(q + 1);
+      __builtin_amdgcn_sched_barrier(0);
+      const int i = 16 * B + q / NC, j0 = 16 * (B + q % NC);
+#pragma unroll
+      for (int e = 0; e < 16; ++e)
+         if (j0 + e > i) x[j0 + e] = fnma(x[i], t[q & 1][e / 2][e % 2], x[j0 + e]);
+      __builtin_amdgcn_sched_barrier(0);
+   }
+}
+
+__device__ __forceinline__ int apply_row(double (&x)[kAppNB], const double (*Tt)[kTtLd], const double* dlv, int kb,
+                                         double small, double inv_u) {
+#pragma clang fp contract(off)
+   apply_rows16<0>(x, Tt);
+   if (kb > 16) apply_rows16<1>(x, Tt);
+   if (kb > 32) apply_rows16<2>(x, Tt);
+   if (kb > 48) apply_rows16<3>(x, Tt);
+   // the same for every row: as scalars, so that the pivots' kinds branch
+   auto dl = [&](int k) { return uniform_value(dlv[k]); };
    bool second = false;  // j is the second column of a 2x2 pivot
 #pragma unroll
    for (int j = 0; j < kAppNB; ++j) {
       if (j >= kb) continue;
       if (second) {
          second = false;
-      } else if (j + 1 < kb && __builtin_isinf(dl[2 * j + 2])) {
+      } else if (j + 1 < kb && __builtin_isinf(dl(2 * j + 2))) {
          const double a1 = x[j], a2 = x[(j + 1) % kAppNB];
-         x[j] = dot2(dl[2 * j], a1, dl[2 * j + 1], a2);
-         x[(j + 1) % kAppNB] = dot2(dl[2 * j + 1], a1, dl[2 * j + 3], a2);
+         x[j] = dot2(dl(2 * j), a1, dl(2 * j + 1), a2);
+         x[(j + 1) % kAppNB] = dot2(dl(2 * j + 1), a1, dl(2 * j + 3), a2);
          second = true;
       } else {
-         apply_dinv1(dl[2 * j], small, x[j]);
+         apply_dinv1(dl(2 * j), small, x[j]);
       }
    }
    int fail = kb;
@@ -229,7 +262,7 @@ __device__ __forceinline__ int bp_block(double (*T)[kAppNB + 1], double* dl, int
 #pragma clang fp contract(off)
    static_assert(kAppNB == 64 && kThreads == 256, "a row per lane, 16 columns per wave");
    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-   auto dmax = [](double p, double q) { return q > p ? q : p; };
+   auto dmax = [](double p, double q) { return __builtin_fmax(p, q); };  // a NaN never wins
    auto imin = [](int p, int q) { return min(p, q); };
    int pos = lane < kb ? lane : -1;
    double t[16], dg = lane < kb ? T[lane][lane] : 0.0;
@@ -252,11 +285,10 @@ __device__ __forceinline__ int bp_block(double (*T)[kAppNB + 1], double* dl, int
       if ((p & 3) == wave) act &= ~(1u << (p >> 2));
    };
    int bad = 0, s = 0;
-   while (s < kb) {
-      double v = -1.0;
+   double v = -1.0;  // largest entry of the lane's row in the wave's active columns
 #pragma unroll
-      for (int u = 0; u < 16; ++u)
-         if (act >> u & 1) v = dmax(v, fabs(t[u]));
+   for (int u = 0; u < 16; ++u) v = dmax(v, fabs(t[u]));
+   while (s < kb) {
       v = wave_reduce(pos >= s ? v : -1.0, dmax);
       if (lane == 0) sc.mx[wave] = v;
       // largest diagonal entry, the smallest position among equal ones (every wave for itself)
@@ -298,12 +330,14 @@ __device__ __forceinline__ int bp_block(double (*T)[kAppNB + 1], double* dl, int
             }
          }
          dg = fnma(lr, br, dg);
+         v = -1.0;
 #pragma unroll
          for (int u = 0; u < 16; ++u)
             if (act >> u & 1) {
                const double bc = lane_value(t[u], p), lc = bc * d0;
                const bool low = pos >= lane_value(pos, 4 * u + wave);
                t[u] = fnma(low ? lr : lc, low ? bc : br, t[u]);
+               v = dmax(v, fabs(t[u]));
             }
          s += 1;
       } else {
@@ -355,6 +389,7 @@ __device__ __forceinline__ int bp_block(double (*T)[kAppNB + 1], double* dl, int
             }
          }
          dg = fnma(l1, r2, fnma(l0, r1, dg));
+         v = -1.0;
 #pragma unroll
          for (int u = 0; u < 16; ++u)
             if (act >> u & 1) {
@@ -362,6 +397,7 @@ __device__ __forceinline__ int bp_block(double (*T)[kAppNB + 1], double* dl, int
                const double k0 = dot2(d0, c1, d1, c2), k1 = dot2(d1, c1, d3, c2);
                const bool low = pos >= lane_value(pos, 4 * u + wave);
                t[u] = fnma(low ? l1 : k1, low ? c2 : r2, fnma(low ? l0 : k0, low ? c1 : r1, t[u]));
+               v = dmax(v, fabs(t[u]));
             }
          s += 2;
       }
@@ -546,7 +582,7 @@ static __global__ __launch_bounds__(kThreads) void k_app_front(const int* __rest
 #pragma clang fp contract(off)
    constexpr int NB = kAppNB;
    __shared__ double T[NB][NB + 1];
-   __shared__ double VS[NB][NB + 1];
+   __shared__ __align__(16) double VS[NB][kTtLd];
    __shared__ double dl[2 * NB];
    __shared__ BpScratch sc;
    __shared__ double red_v[8];
@@ -610,14 +646,13 @@ static __global__ __launch_bounds__(kThreads) void k_app_front(const int* __rest
                Bk[r + (int64_t)j * m] = x[j];
             }
       }
-      for (int k = tid; k < n; k += kThreads) {
+      // (a column per wave, the block's rows over the lanes)
+      for (int k = tid >> 6; k < n; k += kThreads / 64) {
          if (k >= c0 && k < c0 + kb) continue;
-         double x[NB];
-#pragma unroll
-         for (int j = 0; j < NB; ++j) x[j] = (j < kb) ? F[c0 + perm[j] + (int64_t)k * ld] : 0.0;
-#pragma unroll
-         for (int j = 0; j < NB; ++j)
-            if (j < kb) F[c0 + j + (int64_t)k * ld] = x[j];
+         double* col = F + c0 + (int64_t)k * ld;
+         const int j = tid & 63;
+         const double x = j < kb ? col[perm[j]] : 0.0;
+         if (j < kb) col[j] = x;
       }
       {
          int vv = 0, pp = 0;
@@ -642,6 +677,10 @@ static __global__ __launch_bounds__(kThreads) void k_app_front(const int* __rest
       __syncthreads();
       // ---- ApplyN / ApplyT on every other uneliminated row + threshold ----
       if (tid == 0) s_fail = kb;
+      for (int e = tid; e < NB * NB; e += kThreads) {
+         const int j = e & (NB - 1), i = e / NB;
+         if (j > i) VS[i][j] = j < kb ? T[j][i] : 0.0;
+      }
       __syncthreads();
       const double inv_u = 1.0 / u;
       for (int r = tid; r < m; r += kThreads) {
@@ -649,7 +688,7 @@ static __global__ __launch_bounds__(kThreads) void k_app_front(const int* __rest
          double x[NB];
 #pragma unroll
          for (int j = 0; j < NB; ++j) x[j] = (j < kb) ? F[r + (int64_t)(c0 + j) * ld] : 0.0;
-         const int fail = apply_row(x, T, dl, kb, small, inv_u);
+         const int fail = apply_row(x, VS, dl, kb, small, inv_u);
          if (fail < kb) atomicMin(&s_fail, fail);
 #pragma unroll
          for (int j = 0; j < NB; ++j)
@@ -985,13 +1024,17 @@ static __global__ __launch_bounds__(kThreads) void k_lp_perm(int node, int c0, c
       }
       return;
    }
-   const int64_t items = (int64_t)m + n;  // the launch has at least two workgroups
-   for (int64_t it = (int64_t)(blockIdx.x - 1) * kThreads + tid; it < items;
-        it += (int64_t)max(1u, gridDim.x - 1) * kThreads) {
-      double v[NB];
-      if (it < m) {
-         const int r = (int)it;
-         if (r >= c0 && r < c0 + kb) continue;
+   // the launch has at least two workgroups: items of 64 rows (a row per
+   // lane), then items of one fully-summed column (the block's rows over the
+   // lanes), a wave each
+   const int lane = tid & 63;
+   const int64_t nrow = (m + 63) / 64, items = nrow + n;
+   for (int64_t it = (int64_t)(blockIdx.x - 1) * (kThreads / 64) + (tid >> 6); it < items;
+        it += (int64_t)max(1u, gridDim.x - 1) * (kThreads / 64)) {
+      if (it < nrow) {
+         const int r = (int)it * 64 + lane;
+         if (r >= m || (r >= c0 && r < c0 + kb)) continue;
+         double v[NB];
 #pragma unroll
          for (int j = 0; j < NB; ++j) v[j] = (j < kb) ? F[r + (int64_t)(c0 + pm[j]) * ld] : 0.0;
 #pragma unroll
@@ -1001,59 +1044,70 @@ static __global__ __launch_bounds__(kThreads) void k_lp_perm(int node, int c0, c
                w.Bk[r + (int64_t)j * m] = v[j];
             }
       } else {
-         const int k = (int)(it - m);
+         const int k = (int)(it - nrow);
          if (k >= c0 && k < c0 + kb) continue;
-#pragma unroll
-         for (int j = 0; j < NB; ++j) v[j] = (j < kb) ? F[c0 + pm[j] + (int64_t)k * ld] : 0.0;
-#pragma unroll
-         for (int j = 0; j < NB; ++j)
-            if (j < kb) F[c0 + j + (int64_t)k * ld] = v[j];
+         double* col = F + c0 + (int64_t)k * ld;
+         const double x = lane < kb ? col[pm[lane]] : 0.0;
+         if (lane < kb) col[lane] = x;
       }
    }
 }
 
 // ApplyN/ApplyT and the threshold test on the uneliminated rows outside the
-// block: the failed columns so far, then rows c0 + kb .. m - 1.
-static __global__ __launch_bounds__(kThreads) void k_lp_apply(int node, int c0, int par, const IndefDesc* __restrict__ nodes,
-                                                       double* __restrict__ arena, double* __restrict__ wsbase,
-                                                       double u, double small) {
+// block: the failed columns so far, then rows c0 + kb .. m - 1. One wave per
+// workgroup (64 rows, a row per lane): a front of a few thousand rows then
+// spreads over as many CUs as it has such groups. The mirrored entries of the
+// fully-summed rows go out through LDS, a column of 64 per store.
+static __global__ __launch_bounds__(64) void k_lp_apply(int node, int c0, int par, const IndefDesc* __restrict__ nodes,
+                                                 double* __restrict__ arena, double* __restrict__ wsbase, double u,
+                                                 double small) {
 #pragma clang fp contract(off)
    constexpr int NB = kAppNB;
-   __shared__ double T[NB][NB + 1];
+   __shared__ __align__(16) double Tt[NB][kTtLd];
+   __shared__ double tile[NB][NB + 1];
    __shared__ double dl[2 * NB];
-   __shared__ int s_fail;
    const IndefDesc nd = nodes[node];
-   const int m = nd.m, n = nd.n, ld = nd.ld, tid = threadIdx.x;
+   const int m = nd.m, n = nd.n, ld = nd.ld, lane = threadIdx.x;
    const AppWs w = app_ws(wsbase + nd.ws_off, m, n);
    if (w.ST[kStBad]) return;
    const int kb = min(NB, n - c0);
    double* F = arena + nd.off;
-   for (int e = tid; e < kb * kb; e += kThreads) {
-      const int i = e % kb, j = e / kb;
-      T[i][j] = w.TG[i + j * NB];
-   }
-   for (int k = tid; k < 2 * kb; k += kThreads) dl[k] = (par ? w.DL2 : w.DL)[k];
-   if (tid == 0) s_fail = kb;
+#pragma unroll 16
+   for (int i = 0; i < NB; ++i) Tt[i][lane] = (i < lane && lane < kb) ? w.TG[lane + i * NB] : 0.0;
+   for (int k = lane; k < 2 * kb; k += 64) dl[k] = (par ? w.DL2 : w.DL)[k];
    __syncthreads();
+   const auto cols = buf_rsrc(F + (int64_t)c0 * ld, (uint32_t)kb * (uint32_t)ld * 8u);
    const int nf = w.ST[kStNf];
    const double inv_u = 1.0 / u;
    const int64_t items = (int64_t)nf + (m - c0 - kb);
-   for (int64_t it = (int64_t)blockIdx.x * kThreads + tid; it < items; it += (int64_t)gridDim.x * kThreads) {
-      const int r = it < nf ? w.FL[it] : c0 + kb + (int)(it - nf);
+   int fail = kb;
+   for (int64_t it0 = (int64_t)blockIdx.x * 64; it0 < items; it0 += (int64_t)gridDim.x * 64) {
+      const int64_t it = it0 + lane;
+      const bool in = it < items;
+      const int r = !in ? -1 : it < nf ? w.FL[it] : c0 + kb + (int)(it - nf);
+      const uint32_t off = in ? (uint32_t)r * 8u : kOffMask;  // beyond kb columns: zero, dropped
       double x[NB];
 #pragma unroll
-      for (int j = 0; j < NB; ++j) x[j] = (j < kb) ? F[r + (int64_t)(c0 + j) * ld] : 0.0;
-      const int fail = apply_row(x, T, dl, kb, small, inv_u);
-      if (fail < kb) atomicMin(&s_fail, fail);
+      for (int j = 0; j < NB; ++j) x[j] = buf_load_s(cols, off, uniform((uint32_t)(j * ld) * 8u), (double*)nullptr);
+      const int f = apply_row(x, Tt, dl, kb, small, inv_u);
+      if (in) fail = min(fail, f);
 #pragma unroll
-      for (int j = 0; j < NB; ++j)
-         if (j < kb) {
-            F[r + (int64_t)(c0 + j) * ld] = x[j];
-            if (r < n) F[c0 + j + (int64_t)r * ld] = x[j];
+      for (int j = 0; j < NB; ++j) buf_store_s(cols, off, uniform((uint32_t)(j * ld) * 8u), x[j]);
+      const unsigned long long sum_rows = __ballot(in && r < n);
+      if (sum_rows) {
+         __syncthreads();
+#pragma unroll
+         for (int j = 0; j < NB; ++j) tile[lane][j] = x[j];
+         __syncthreads();
+         for (unsigned long long b = sum_rows; b; b &= b - 1) {
+            const int k = (int)__builtin_ctzll(b);
+            const int row = lane_value(r, k);
+            if (lane < kb) F[c0 + lane + (int64_t)row * ld] = tile[k][lane];
          }
+      }
    }
-   __syncthreads();
-   if (tid == 0 && s_fail < kb) atomicMin(&w.ST[kStFail], s_fail);
+   fail = wave_reduce(fail, [](int p, int q) { return min(p, q); });
+   if (lane == 0 && fail < kb) atomicMin(&w.ST[kStFail], fail);
 }
 
 // Passed count of the block, L11 of the passed columns, their D^{-1} and
@@ -1099,7 +1153,9 @@ static __global__ __launch_bounds__(kThreads) void k_lp_finish(int node, int c0,
    }
 }
 
-constexpr int kLpTile = 128;  // tile of the multi-workgroup fully-summed update
+// tile of the multi-workgroup fully-summed update: 64 x 64, 4 x 4 entries a
+// thread (128 x 128 left most CUs idle on fronts of few fully-summed columns)
+constexpr int kLpTile = 64;
 
 // Entries of k_lp_update by mode: 0 all, 1 only those of the next block's
 // diagonal block (row and column index positions in [nf, nf + kb2)), 2 all
@@ -1146,7 +1202,9 @@ static __global__ __launch_bounds__(kThreads) void k_lp_update(int node, int c0,
    const int64_t nt = mode == 1 ? (t1 > t0 ? 3 : 1) : ntiles;
    for (int k = tid; k < 2 * kb; k += kThreads) dl[k] = (par ? w.DL2 : w.DL)[k];
    const int lo = c0 + npass, hi = c0 + kb;  // failed block columns
-   const int tr8 = tid & 15, tc8 = tid >> 4;
+   // thread (tr, tc): rows tr + 16 a and columns tc + 16 b of the tile
+   constexpr int R = TT / 16;
+   const int tr16 = tid & 15, tc16 = tid >> 4;
    for (int64_t t = blockIdx.x; t < nt; t += gridDim.x) {
       int tc = 0, tr = 0;
       if (mode == 1) {
@@ -1163,7 +1221,7 @@ static __global__ __launch_bounds__(kThreads) void k_lp_update(int node, int c0,
       const int R0 = tr * TT, S0 = tc * TT;
       if (npass == 0 && !(R0 < nf && R0 + TT > nf_old) && !(S0 < nf && S0 + TT > nf_old)) continue;
       __syncthreads();
-      {
+      if (tid < 2 * TT) {
          const int k = (tid < TT ? R0 : S0) + (tid & (TT - 1));
          const int lim = tid < TT ? nr : nu;
          int v = -1;
@@ -1187,15 +1245,15 @@ static __global__ __launch_bounds__(kThreads) void k_lp_update(int node, int c0,
          }
          Bs[p][i] = v;
       }
-      double acc[8][8];
+      double acc[R][R];
 #pragma unroll
-      for (int b = 0; b < 8; ++b) {
-         const int s = cidx[tc8 * 8 + b];
+      for (int b = 0; b < R; ++b) {
+         const int s = cidx[tc16 + 16 * b];
 #pragma unroll
-         for (int a = 0; a < 8; ++a) {
-            const int r = ridx[tr8 * 8 + a];
+         for (int a = 0; a < R; ++a) {
+            const int r = ridx[tr16 + 16 * a];
             double x = 0.0;
-            if (r >= 0 && s >= 0 && r >= s && lp_keep(mode, R0 + tr8 * 8 + a, S0 + tc8 * 8 + b, nf, kb2)) {
+            if (r >= 0 && s >= 0 && r >= s && lp_keep(mode, R0 + tr16 + 16 * a, S0 + tc16 + 16 * b, nf, kb2)) {
                if (s >= lo && s < hi)
                   x = w.Bk[r + (int64_t)(s - c0) * m];
                else if (r >= lo && r < hi)
@@ -1208,23 +1266,23 @@ static __global__ __launch_bounds__(kThreads) void k_lp_update(int node, int c0,
       }
       __syncthreads();
       for (int p = 0; p < npass; ++p) {
-         double av[8], bv[8];
+         double av[R], bv[R];
 #pragma unroll
-         for (int a = 0; a < 8; ++a) av[a] = As[p][tr8 * 8 + a];
+         for (int a = 0; a < R; ++a) av[a] = As[p][tr16 + 16 * a];
 #pragma unroll
-         for (int b = 0; b < 8; ++b) bv[b] = Bs[p][tc8 * 8 + b];
+         for (int b = 0; b < R; ++b) bv[b] = Bs[p][tc16 + 16 * b];
 #pragma unroll
-         for (int a = 0; a < 8; ++a)
+         for (int a = 0; a < R; ++a)
 #pragma unroll
-            for (int b = 0; b < 8; ++b) acc[a][b] = fnma(av[a], bv[b], acc[a][b]);
+            for (int b = 0; b < R; ++b) acc[a][b] = fnma(av[a], bv[b], acc[a][b]);
       }
 #pragma unroll
-      for (int b = 0; b < 8; ++b) {
-         const int s = cidx[tc8 * 8 + b];
+      for (int b = 0; b < R; ++b) {
+         const int s = cidx[tc16 + 16 * b];
 #pragma unroll
-         for (int a = 0; a < 8; ++a) {
-            const int r = ridx[tr8 * 8 + a];
-            if (r >= 0 && s >= 0 && r >= s && lp_keep(mode, R0 + tr8 * 8 + a, S0 + tc8 * 8 + b, nf, kb2)) {
+         for (int a = 0; a < R; ++a) {
+            const int r = ridx[tr16 + 16 * a];
+            if (r >= 0 && s >= 0 && r >= s && lp_keep(mode, R0 + tr16 + 16 * a, S0 + tc16 + 16 * b, nf, kb2)) {
                F[r + (int64_t)s * ld] = acc[a][b];
                if (r < n && r > s) F[s + (int64_t)r * ld] = acc[a][b];
             }

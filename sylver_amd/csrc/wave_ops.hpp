@@ -34,6 +34,14 @@ __device__ __forceinline__ double lane_value(double v, int lane) {
    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
 
+// v, the same in every active lane, as a scalar.
+__device__ __forceinline__ double uniform_value(double v) {
+   const long long u = __double_as_longlong(v);
+   const int lo = __builtin_amdgcn_readfirstlane((int)(u & 0xffffffff));
+   const int hi = __builtin_amdgcn_readfirstlane((int)(u >> 32));
+   return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+
 // Reduction over the wave by `op` (associative, idempotent): row scans, then
 // the rows' last lanes onward; lane 63 ends with the result.
 template <typename V, typename Op>
