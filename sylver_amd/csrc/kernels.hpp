@@ -1910,7 +1910,6 @@ constexpr int kChainMaxPolls = 1 << 20;
 constexpr unsigned long long kYEmpty = 0x7FF4DEADBEEF0000ull;
 constexpr int kChainThreads = 512;  // 8 waves: one 16-row tile of the block each
 
-
 template <typename T, bool BWD>
 __global__ __launch_bounds__(kChainThreads) void k_chain(const ChainTask* __restrict__ tasks,
                                                          const NodeDesc* __restrict__ nodes,
@@ -1920,14 +1919,15 @@ __global__ __launch_bounds__(kChainThreads) void k_chain(const ChainTask* __rest
                                                          double* __restrict__ ybuf, const double* __restrict__ part,
                                                          int* __restrict__ err, const int4* __restrict__ cgch,
                                                          const int* __restrict__ cmap, const double* __restrict__ b,
-                                                         int ldb) {
+                                                         int ldb, int gch) {
    constexpr int KU = kNB / 4;                         // k-steps of the 16x16x4 MFMA over 128
    constexpr int YU = kNB * 16 / kChainThreads;        // staged y values per thread
    constexpr uint32_t ES = sizeof(T);
    typedef typename Mfma<T>::acc_t acc_t;
    __shared__ T ys[kNB * 16];  // staged y (rounded to T, as the products use it)
    __shared__ double xg[BWD ? 1 : kNB * 16];  // forward: the block's gathered x
-   const ChainTask t = tasks[blockIdx.x];
+   const int tix = (int)blockIdx.x / gch;  // the chunks of a task are neighbours
+   const ChainTask t = tasks[tix];
    const NodeDesc nd = nodes[t.node];
    const int m = nd.m, n = nd.n, ld = nd.ld, rows = t.r1 - t.r0;
    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -1989,8 +1989,9 @@ __global__ __launch_bounds__(kChainThreads) void k_chain(const ChainTask* __rest
          for (int u = 0; u < KU; ++u) av[u] = buf_load(frs, lo + (uint32_t)u * step, (T*)nullptr);
       }
    };
-   for (int c0 = 0, ci = 0; c0 < nrhs; c0 += 16, ++ci) {
-      const int nc = min(16, nrhs - c0);
+   const int ci0 = (int)blockIdx.x - tix * gch;
+   for (int ci = ci0; ci < nch; ci += gch) {
+      const int c0 = 16 * ci, nc = min(16, nrhs - c0);
       // the block's x: backward from the solution (the forward's y on the
       // pivot rows), forward gathered from b and the children
       double xv[4];
@@ -2001,7 +2002,7 @@ __global__ __launch_bounds__(kChainThreads) void k_chain(const ChainTask* __rest
             xv[v] = (o < rows && r < nc) ? xsol[sidx[v] + (int64_t)(c0 + r) * ldsol] : 0.0;
          }
       } else {
-         if (c0 > 0) __syncthreads();  // the previous chunk is done with xg
+         if (ci > ci0) __syncthreads();  // the previous chunk is done with xg
          chain_gather<kChainThreads>(xg, t, nd, nodes, cgch, rlist, cmap, xloc, b, ldb, nrhs, c0, nc, 0, rows);
 #pragma unroll
          for (int v = 0; v < 4; ++v) xv[v] = xg[(wave * 16 + Mfma<T>::row(lane, v)) * 16 + r];
@@ -2108,6 +2109,274 @@ __global__ __launch_bounds__(kChainThreads) void k_chain(const ChainTask* __rest
          }
       }
    }
+}
+
+// k_chain for few right-hand sides, in chunks of NR = 1 or 2. What bounds a
+// chain step is the latency of its two products on one CU: as 16-column MFMA
+// tiles they take 3.4 us in FP64 (1.7 us in FP32) however few columns there
+// are, as vector sums in FP64 on the VALU 0.2 us a column. And no wave waits
+// for another before the diagonal step: each polls for the entries of y that
+// it multiplies, straight into registers, and keeps its partial sums over all
+// the blocks.
+//   Forward: thread (i, q) has row i of the block and the columns 32 q ..
+//   32 q + 31 of a tile; its wave's 32 entries of y come from the lanes that
+//   polled them by v_readlane.
+//   Backward: wave w has the block's columns 16 w .. 16 w + 15 and lane l the
+//   rows 2 l, 2 l + 1 of a tile, so that a column of L is one contiguous load.
+// The diagonal step is the same in both: the partial sums meet in LDS, x is
+// multiplied by the block's stored inverse (thread (i, q): columns 32 q ...),
+// the four partial results are summed by thread (i, c) of column c, which
+// publishes y. Exchange slot of a block and chunk: NR x kNB doubles, a column
+// after the other. Same tasks, order and bounded waits as k_chain. (Four
+// columns a workgroup spill in FP64 and were slower than two chunks of two.)
+//
+// Chunks are chains of their own, side by side in the launch (the chunks of a
+// task are neighbours in dispatch order, so that a tile of L is read once
+// into the caches); k_chain went through them in one workgroup, one after the
+// other. 33 columns, 53 x 50 x 47 in FP32 with refinement: 11.2 -> 9.0 ms;
+// 80^3 in FP64: 24.6 -> 19.9 ms.
+// The line at eight columns: whole solves in us, 16-column MFMA tiles ->
+// chunks of 1 (1 column) or 2,
+//   columns              1           2           4           8           12
+//   80^3 FP64    5281->3113  5643->4105  6528->5308  8120->7676  9878->10291
+//   61x60x59 FP64 2822->1604  2983->2155  3337->2547  3960->3421  4731->4463
+//   53x50x47 FP32 3511->2554  3644->3233  3908->3465  4351->4102  4838->4895
+//   23x21x20 FP64  601-> 447   575-> 452   635-> 518   730-> 604   833-> 712
+// (the tiles' cost hardly grows up to 16 columns, the chunks' reads of L do).
+constexpr int kChainFewRhs = 8;
+// Columns of a chunk, chunks, and workgroups a task (k_chain loops over the
+// chunks beyond; the bound keeps the launch below 2^31 threads).
+struct ChainShape {
+   int width, chunks, grid;
+};
+inline ChainShape chain_shape(int nrhs, int ntask) {
+   const int w = nrhs == 1 ? 1 : nrhs <= kChainFewRhs ? 2 : 16, nch = (nrhs + w - 1) / w;
+   return {w, nch, w < 16 ? nch : std::min(nch, std::max(1, (1 << 22) / std::max(ntask, 1)))};
+}
+
+// Device-scope loads of this lane's entries of a block's y until all are
+// written; src[u] for u < N, only those with `need` bit set.
+template <int N>
+__device__ __forceinline__ void chain_poll(const double* const (&src)[N], unsigned need, double (&yv)[N],
+                                           int* __restrict__ err) {
+   for (int p = 0; need; ++p) {
+#pragma unroll
+      for (int u = 0; u < N; ++u)
+         if (need & (1u << u)) {
+            const double v = __hip_atomic_load(src[u], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (__builtin_bit_cast(unsigned long long, v) != kYEmpty) {
+               yv[u] = v;
+               need &= ~(1u << u);
+            }
+         }
+      if (!need) break;
+      if (p >= kChainMaxPolls ||
+          ((p & 255) == 255 && __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)) {
+         __hip_atomic_fetch_add(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+         break;
+      }
+      __builtin_amdgcn_s_sleep(1);
+   }
+}
+
+template <typename T, bool BWD, int NR>
+__global__ __launch_bounds__(kChainThreads) void k_chain_few(
+    const ChainTask* __restrict__ tasks, const NodeDesc* __restrict__ nodes, const T* __restrict__ arena,
+    const T* __restrict__ dinvs, const int* __restrict__ rlist, double* __restrict__ xloc, double* __restrict__ xsol,
+    int ldsol, int nrhs, double* __restrict__ ybuf, const double* __restrict__ part, int* __restrict__ err,
+    const int4* __restrict__ cgch, const int* __restrict__ cmap, const double* __restrict__ b, int ldb, int nch) {
+   static_assert(kChainThreads == 512 && kNB == 128 && NR <= 4, "four threads a row, a column of y each");
+   constexpr uint32_t ES = sizeof(T);
+   constexpr int KQ = kNB / 4;  // columns of a thread
+   __shared__ double xg[NR][kNB], ys[NR][kNB], red[4][NR][kNB];
+   __shared__ double lanes[BWD ? kNB * 65 : 1];  // backward: lane sums of every column
+   const int tix = (int)blockIdx.x / nch, ci = (int)blockIdx.x - tix * nch;  // the chunks of a task are neighbours
+   const int c0 = ci * NR, nc = min(NR, nrhs - c0);
+   const ChainTask t = tasks[tix];
+   const NodeDesc nd = nodes[t.node];
+   const int m = nd.m, n = nd.n, ld = nd.ld, rows = t.r1 - t.r0;
+   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+   const int i = tid & (kNB - 1), q = __builtin_amdgcn_readfirstlane(tid >> 7);
+   const bool mine = i < rows && q < nc;  // this thread has row i of the chunk's column q of x and y
+   double* xl = xloc + nd.solve_off * nrhs + (int64_t)c0 * m;
+   auto yslot = [&](int blk) { return ybuf + ((int64_t)(t.flag0 + blk) * nch + ci) * (NR * kNB); };
+   const bool diag = t.blk < t.nb;
+   const int ntile = BWD ? t.nb - 1 - t.blk : min(t.blk, t.nb);
+   const uint32_t fbytes = (uint32_t)n * (uint32_t)ld * ES;
+   const __amdgpu_buffer_rsrc_t frs = buf_rsrc(arena + nd.off, fbytes);
+   // tile s: forward columns kb0 + 32 q + u of row r0 + i; backward rows
+   // kb0 + 2 l, + 1 of columns r0 + 16 w + u (rows at or beyond n meet zeros of y)
+   typedef T pair __attribute__((ext_vector_type(2)));
+   T av[BWD ? 1 : KQ];
+   pair ap[BWD ? 16 : 1];
+   auto load_tile = [&](int s) {
+      const int kb0 = (BWD ? t.nb - 1 - s : s) * kNB;
+      if constexpr (BWD) {
+         const uint32_t lo = (uint32_t)(kb0 + 2 * lane) * ES;
+#pragma unroll
+         for (int u = 0; u < 16; ++u) {
+            const int col = wave * 16 + u;
+            const uint32_t o = col < rows ? lo + (uint32_t)((t.r0 + col) * ld) * ES : fbytes;
+            if constexpr (sizeof(T) == 8) {
+               const auto raw = __builtin_amdgcn_raw_buffer_load_b128(frs, (int)o, 0, 0);
+               __builtin_memcpy(&ap[u], &raw, 16);
+            } else {
+               const auto raw = __builtin_amdgcn_raw_buffer_load_b64(frs, (int)o, 0, 0);
+               __builtin_memcpy(&ap[u], &raw, 8);
+            }
+         }
+      } else {
+         const uint32_t lo = i < rows ? (uint32_t)(t.r0 + i + (kb0 + KQ * q) * ld) * ES : fbytes;
+#pragma unroll
+         for (int u = 0; u < KQ; ++u) av[u] = buf_load(frs, lo + (uint32_t)(u * ld) * ES, (T*)nullptr);
+      }
+   };
+   if (ntile > 0) load_tile(0);
+   // rows of the block's inverse: up front, or after the tile loop where the
+   // sums of several columns leave no registers for them
+   constexpr bool kInvEarly = !BWD || NR == 1;
+   T mv[KQ];
+   auto load_inv = [&]() {
+      const uint32_t mbytes = (uint32_t)(rows * rows) * ES;
+      const __amdgpu_buffer_rsrc_t mrs = buf_rsrc(dinvs + nd.dinv_off + (int64_t)t.blk * kNB * kNB, mbytes);
+      const uint32_t lo = i < rows ? (uint32_t)(i + KQ * q * rows) * ES : mbytes;
+#pragma unroll
+      for (int u = 0; u < KQ; ++u) mv[u] = buf_load(mrs, lo + (uint32_t)(u * rows) * ES, (T*)nullptr);
+   };
+   if (kInvEarly && diag) load_inv();
+   const int grow = t.r0 + i;
+   const int sidx = (mine && diag) ? rlist[nd.rlist_off + grow] - 1 : 0;
+   // the block's x: forward b and then the children's rows in list order,
+   // backward the solution (the forward's y) minus the contribution block's product
+   double xv = 0.0;
+   if constexpr (BWD) {
+      if (mine) {
+         xv = xsol[sidx + (int64_t)(c0 + q) * ldsol];
+         if (t.cbn > 0) {
+            const double* pp = part + ((int64_t)(t.cb0 + (grow >> 6) * t.cbn) * 64 + (grow & 63)) * nrhs + c0 + q;
+            const int64_t st = (int64_t)64 * nrhs;
+            double sum = 0.0;  // slots summed in order, loads eight at a time
+            int k = 0;
+            for (; k + 8 <= t.cbn; k += 8) {
+               double pv[8];
+#pragma unroll
+               for (int e = 0; e < 8; ++e) pv[e] = pp[(k + e) * st];
+#pragma unroll
+               for (int e = 0; e < 8; ++e) sum += pv[e];
+            }
+            for (; k < t.cbn; ++k) sum += pp[k * st];
+            xv -= sum;
+         }
+      }
+   } else {
+      if (q < NR) xg[q][i] = (mine && diag) ? b[sidx + (int64_t)(c0 + q) * ldb] : 0.0;
+      for (int g = t.g0; g < t.g0 + t.gn; ++g) {
+         const int4 cg = cgch[g];
+         const NodeDesc cn = nodes[cg.x];
+         const int* cm = cmap + cn.cmap_off;
+         const double* cx = xloc + cn.solve_off * nrhs + (int64_t)c0 * cn.m + cn.n;
+         __syncthreads();
+         if (q < nc)
+            for (int e = cg.y + i; e < cg.z; e += kNB) xg[q][cm[e] - t.r0] += cx[e + (int64_t)q * cn.m];
+      }
+      __syncthreads();
+      if (q < NR) xv = xg[q][i];
+   }
+   double acc[BWD ? 16 : 1][NR];
+#pragma unroll
+   for (int u = 0; u < (BWD ? 16 : 1); ++u)
+#pragma unroll
+      for (int c = 0; c < NR; ++c) acc[u][c] = 0.0;
+   for (int s = 0; s < ntile; ++s) {
+      const int kblk = BWD ? t.nb - 1 - s : s, kbk = min(kNB, n - kblk * kNB);
+      const double* slot = yslot(kblk);
+      if constexpr (BWD) {
+         const double* src[2 * NR];
+         double yv[2 * NR];
+         unsigned need = 0;
+#pragma unroll
+         for (int u = 0; u < 2 * NR; ++u) {
+            const int l = 2 * lane + (u & 1), c = u >> 1;
+            src[u] = slot + c * kNB + l;
+            yv[u] = 0.0;
+            if (l < kbk && c < nc) need |= 1u << u;
+         }
+         chain_poll(src, need, yv, err);
+#pragma unroll
+         for (int u = 0; u < 16; ++u)
+#pragma unroll
+            for (int c = 0; c < NR; ++c)
+               acc[u][c] = fma((double)ap[u][1], yv[2 * c + 1], fma((double)ap[u][0], yv[2 * c], acc[u][c]));
+      } else {
+         constexpr int PU = (KQ * NR + 63) / 64;
+         const double* src[PU];
+         double yv[PU];
+         unsigned need = 0;
+#pragma unroll
+         for (int u = 0; u < PU; ++u) {
+            const int e = lane + 64 * u, l = KQ * q + (e & (KQ - 1)), c = e / KQ;
+            src[u] = slot + c * kNB + l;
+            yv[u] = 0.0;
+            if (l < kbk && c < nc) need |= 1u << u;
+         }
+         chain_poll(src, need, yv, err);
+#pragma unroll
+         for (int c = 0; c < NR; ++c) {
+            double a0 = 0.0, a1 = 0.0;  // two chains a tile
+#pragma unroll
+            for (int k = 0; k < KQ; k += 2) {
+               a0 = fma((double)av[k], lane_bcast(yv[(c * KQ + k) / 64], (c * KQ + k) % 64), a0);
+               a1 = fma((double)av[k + 1], lane_bcast(yv[(c * KQ + k + 1) / 64], (c * KQ + k + 1) % 64), a1);
+            }
+            acc[0][c] += a0 + a1;
+         }
+      }
+      if (s + 1 < ntile) load_tile(s + 1);
+   }
+   if (ntile > 0) {
+      if constexpr (BWD) {
+#pragma unroll
+         for (int c = 0; c < NR; ++c) {
+            if (c > 0) __syncthreads();  // the previous column's sums are read
+#pragma unroll
+            for (int u = 0; u < 16; ++u) lanes[(wave * 16 + u) * 65 + lane] = acc[u][c];
+            __syncthreads();
+            double sum = 0.0;
+#pragma unroll
+            for (int e = 0; e < 16; ++e) sum += lanes[i * 65 + q * 16 + e];
+            red[q][c][i] = sum;
+         }
+      } else {
+#pragma unroll
+         for (int c = 0; c < NR; ++c) red[q][c][i] = acc[0][c];
+      }
+      __syncthreads();
+      if (q < NR) xv -= (red[0][q][i] + red[1][q][i]) + (red[2][q][i] + red[3][q][i]);
+   }
+   if (!diag) {
+      if (mine) xl[grow + (int64_t)q * m] = xv;
+      return;
+   }
+   if (!kInvEarly) load_inv();
+   if (q < NR) ys[q][i] = mine ? xv : 0.0;
+   __syncthreads();  // and red is read
+#pragma unroll
+   for (int c = 0; c < NR; ++c) {
+      double a0 = 0.0, a1 = 0.0;
+#pragma unroll
+      for (int u = 0; u < KQ; u += 2) {
+         a0 = fma((double)mv[u], ys[c][KQ * q + u], a0);
+         a1 = fma((double)mv[u + 1], ys[c][KQ * q + u + 1], a1);
+      }
+      red[q][c][i] = a0 + a1;
+   }
+   __syncthreads();
+   if (!mine) return;
+   const double y = (red[0][q][i] + red[1][q][i]) + (red[2][q][i] + red[3][q][i]);
+   __hip_atomic_store(yslot(t.blk) + q * kNB + i, y, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+   // the front's solve vector and the solution (read by later launches)
+   xl[grow + (int64_t)q * m] = y;
+   xsol[sidx + (int64_t)(c0 + q) * ldsol] = y;
 }
 
 static __global__ void k_fill_y(unsigned long long* p, int64_t n) {

@@ -1501,22 +1501,30 @@ void run_solve_program(const DevicePlan* P, DeviceFactors* F, const std::vector<
             if (L.count > 0) k_bwd_cbr<<<g, bl, 0, s>>>(tk, P->d_nodes, F->d_part_cb, F->d_xloc, nrhs);
             break;
          case L_CLEAR: {
-            const int64_t ny = P->chain_flags * ((nrhs + 15) / 16) * kNB * 16;
+            const ChainShape c = chain_shape(nrhs, 1);
+            const int64_t ny = P->chain_flags * c.chunks * c.width * kNB;
             k_fill_y<<<dim3((unsigned)((ny + kThreads - 1) / kThreads)), bl, 0, s>>>(
                 reinterpret_cast<unsigned long long*>(F->d_ybuf), ny);
             break;
          }
          case L_FCHAIN:
-            k_chain<T, false><<<g, dim3(kChainThreads), 0, s>>>(P->d_ctask + L.off, P->d_nodes, arena, dinv,
-                                                                P->d_rlist, F->d_xloc, xsol, n, nrhs, F->d_ybuf,
-                                                                nullptr, F->d_chain, P->d_cgch, P->d_cmap, b, n);
+         case L_BCHAIN: {
+            const bool bwd = L.kind == L_BCHAIN;
+            const ChainShape c = chain_shape(nrhs, L.count);
+            auto chain = [&](auto kernel) {
+               kernel<<<dim3(L.count * c.grid), dim3(kChainThreads), 0, s>>>(
+                   P->d_ctask + L.off, P->d_nodes, arena, bwd ? dinvT : dinv, P->d_rlist, F->d_xloc, xsol, n, nrhs,
+                   F->d_ybuf, bwd ? F->d_part_cb : nullptr, F->d_chain, P->d_cgch, P->d_cmap, bwd ? nullptr : b,
+                   bwd ? 0 : n, c.grid);
+            };
+            if (c.width == 1)
+               bwd ? chain(k_chain_few<T, true, 1>) : chain(k_chain_few<T, false, 1>);
+            else if (c.width == 2)
+               bwd ? chain(k_chain_few<T, true, 2>) : chain(k_chain_few<T, false, 2>);
+            else
+               bwd ? chain(k_chain<T, true>) : chain(k_chain<T, false>);
             break;
-         case L_BCHAIN:
-            k_chain<T, true><<<g, dim3(kChainThreads), 0, s>>>(P->d_ctask + L.off, P->d_nodes, arena, dinvT,
-                                                               P->d_rlist, F->d_xloc, xsol, n, nrhs, F->d_ybuf,
-                                                               F->d_part_cb, F->d_chain, P->d_cgch, P->d_cmap,
-                                                               nullptr, 0);
-            break;
+         }
          default:  // L_SYNC
             break;
       }
