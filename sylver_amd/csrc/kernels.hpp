@@ -2144,14 +2144,20 @@ __global__ __launch_bounds__(kChainThreads) void k_chain(const ChainTask* __rest
 //   23x21x20 FP64  601-> 447   575-> 452   635-> 518   730-> 604   833-> 712
 // (the tiles' cost hardly grows up to 16 columns, the chunks' reads of L do).
 constexpr int kChainFewRhs = 8;
-// Columns of a chunk, chunks, and workgroups a task (k_chain loops over the
-// chunks beyond; the bound keeps the launch below 2^31 threads).
+// Columns of a chunk, chunks, and workgroups a task or front (the MFMA kernels
+// loop over the chunks beyond; the bound keeps the launch below 2^31 threads).
 struct ChainShape {
    int width, chunks, grid;
 };
-inline ChainShape chain_shape(int nrhs, int ntask) {
-   const int w = nrhs == 1 ? 1 : nrhs <= kChainFewRhs ? 2 : 16, nch = (nrhs + w - 1) / w;
+inline ChainShape chunk_shape(int nrhs, int w, int ntask) {
+   const int nch = (nrhs + w - 1) / w;
    return {w, nch, w < 16 ? nch : std::min(nch, std::max(1, (1 << 22) / std::max(ntask, 1)))};
+}
+inline ChainShape chain_shape(int nrhs, int ntask) {
+   return chunk_shape(nrhs, nrhs == 1 ? 1 : nrhs <= kChainFewRhs ? 2 : 16, ntask);
+}
+inline ChainShape small_shape(int nrhs, int ntask) {
+   return chunk_shape(nrhs, nrhs <= 2 ? nrhs : nrhs <= kChainFewRhs ? 4 : 16, ntask);
 }
 
 // Device-scope loads of this lane's entries of a block's y until all are
@@ -2414,7 +2420,8 @@ __device__ inline typename Mfma<T>::acc_t mma_small(const T* __restrict__ A, int
 // m <= 256) in a sweep. Forward: y = inv(L11) x[0:n] to the solution and
 // x[n:m] -= L21 y. Backward: x[0:n] -= L21^T x[n:m], then inv(L11)^T x[0:n]
 // to the solution. The leaf levels hold thousands of such fronts: this
-// kernel keeps its register use low to run several workgroups per CU.
+// kernel keeps its register use low to run several workgroups per CU. Beyond
+// 16 columns the chunks are workgroups of their own (blockIdx.y, gch of them).
 template <typename T, bool BWD>
 __global__ __launch_bounds__(kThreads) void k_solve_small(const int* __restrict__ list,
                                                           const NodeDesc* __restrict__ nodes,
@@ -2424,7 +2431,7 @@ __global__ __launch_bounds__(kThreads) void k_solve_small(const int* __restrict_
                                                           double* __restrict__ xloc,
                                                           double* __restrict__ xsol, int ldsol, int nrhs,
                                                           const double* __restrict__ b, int ldb,
-                                                          const int* __restrict__ cmap, int mrows) {
+                                                          const int* __restrict__ cmap, int mrows, int gch) {
    // LDS sized by the launch to its largest front: x (mrows x 16, mrows =
    // the largest m rounded up to 16, at most 2 kNB) then y (kNB x 16 at
    // most, the largest n); small leaf fronts then fit many workgroups per CU
@@ -2438,7 +2445,7 @@ __global__ __launch_bounds__(kThreads) void k_solve_small(const int* __restrict_
    double* xl = xloc + nd.solve_off * nrhs;
    const T* Mk = dinvs + nd.dinv_off;
    const T* F = arena + nd.off;
-   for (int c0 = 0; c0 < nrhs; c0 += 16) {
+   for (int c0 = 16 * (int)blockIdx.y; c0 < nrhs; c0 += 16 * gch) {
       const int nc = min(16, nrhs - c0);
       __syncthreads();
       // the front's x, gathered here. Backward: every row from the solution.
@@ -2514,6 +2521,231 @@ __global__ __launch_bounds__(kThreads) void k_solve_small(const int* __restrict_
          }
       }
    }
+}
+
+// k_solve_small for chunks of NR = 1, 2 or 4 columns, up to kChainFewRhs. What
+// bounds a level of small fronts is the chain of dependent loads of one
+// front: row map, b, each child's map and rows, then batch after batch of L
+// for 16-column MFMA tiles. Here the products are vector sums in FP64 spread
+// over all 256 threads, whatever the front's size: P = 16, 32, .. 256 threads
+// for the rows, 256 / P groups of columns. The first columns of the stored
+// inverse (backward: of L21) are loaded before the gather, the next batch
+// before a batch is used, and a child's rows before those of the one before
+// it are added. Average of a forward launch, MFMA tiles -> here: 100 x 100
+// FP64, 1 column 14.0 -> 6.8 us; 701 x 523 FP32 28.5 -> 12.1 us;
+// 47 x 39 x 31 FP64, 3 columns 25.5 -> 14.1 us. Whole solves of 53 x 50 x 47
+// FP32: 1 column 2554 -> 2210 us, 4 columns 3465 -> 3267 us, 8 columns 4102 ->
+// 3959 us (the chains being k_chain_few on both sides); 80^3 FP64, 8 columns:
+// 7676 -> 7709 us with chunks of four, 7883 us with chunks of two.
+template <typename T>
+__device__ __forceinline__ void few_load(T (&a)[16], __amdgpu_buffer_rsrc_t rs, uint32_t vo, uint32_t stride, int k,
+                                         int K) {
+#pragma unroll
+   for (int u = 0; u < 16; u += 4)
+      if (k + u < K)
+#pragma unroll
+         for (int e = 0; e < 4; ++e) a[u + e] = buf_load_s(rs, vo, (uint32_t)(k + u + e) * stride, (T*)nullptr);
+}
+
+// acc[c] += sum over k < K of A[k] v[c * vs + k], K a multiple of four,
+// A[k] at byte vo + k * stride (zero out of range), A[0..15] loaded in a
+template <typename T, int NR>
+__device__ __forceinline__ void few_rows(T (&a)[16], __amdgpu_buffer_rsrc_t rs, uint32_t vo, uint32_t stride, int K,
+                                         const double* v, int vs, double (&acc)[NR]) {
+   for (int k = 0; k < K; k += 16) {
+      T nx[16];
+      few_load(nx, rs, vo, stride, k + 16, K);
+#pragma unroll
+      for (int u = 0; u < 16; u += 4)
+         if (k + u < K)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+               for (int c = 0; c < NR; ++c) acc[c] = fma((double)a[u + e], v[c * vs + k + u + e], acc[c]);
+#pragma unroll
+      for (int u = 0; u < 16; ++u) a[u] = nx[u];
+   }
+}
+
+template <typename T, bool BWD, int NR>
+__global__ __launch_bounds__(kThreads) void k_solve_small_few(
+    const int* __restrict__ list, const NodeDesc* __restrict__ nodes, const T* __restrict__ arena,
+    const T* __restrict__ dinvs, const int* __restrict__ rlist, double* __restrict__ xloc,
+    double* __restrict__ xsol, int ldsol, int nrhs, const double* __restrict__ b, int ldb,
+    const int* __restrict__ cmap, int nch) {
+   static_assert(kThreads == 256 && kNB == 128, "a thread a row of the front");
+   constexpr uint32_t ES = sizeof(T), kOut = 1u << 30;
+   constexpr int VK = 16 / (int)ES, RS = 4 * VK;  // backward: rows of a load and of a wave's step
+   __shared__ double x1[NR][kNB], x2[NR][2 * kNB], ys[NR][kNB], red[NR][kThreads];
+   const int tix = (int)blockIdx.x / nch, ci = (int)blockIdx.x - tix * nch;  // the chunks of a front are neighbours
+   const int c0 = ci * NR, nc = min(NR, nrhs - c0);
+   const NodeDesc nd = nodes[list[tix]];
+   const int m = nd.m, n = nd.n, ld = nd.ld, q = m - n;
+   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+   const __amdgpu_buffer_rsrc_t mrs = buf_rsrc(dinvs + nd.dinv_off, (uint32_t)(n * n) * ES);
+   // rows n .. of the columns [0, n): a column index of n or more is out of range
+   const __amdgpu_buffer_rsrc_t frs =
+       BWD ? buf_rsrc(arena + nd.off, (uint32_t)(n * ld) * ES) : buf_rsrc(arena + nd.off + n, (uint32_t)(n * ld - n) * ES);
+   const int gi = tid < (BWD ? m : n) ? rlist[nd.rlist_off + tid] - 1 : -1;
+   // columns of a group: a multiple of four, so that the groups' columns end
+   // at most at 128, where x and y are zero beyond n
+   auto lg_rows = [](int rows) { return rows <= 16 ? 4 : rows <= 32 ? 5 : rows <= 64 ? 6 : rows <= 128 ? 7 : 8; };
+   auto group_cols = [&](int lg) { return 4 * ((n + (1024 >> lg) - 1) >> (10 - lg)); };
+   const int lgp = lg_rows(n), K1 = group_cols(lgp), i1 = tid & ((1 << lgp) - 1), g1 = tid >> lgp;
+   const uint32_t vo1 = i1 < n ? (uint32_t)(i1 + g1 * K1 * n) * ES : kOut;
+   T a[16];
+   // backward: wave w has 16 columns (lane & 15) of L21 and every fourth, second
+   // or each step of RS rows, by the number of column tiles; rows from n
+   // rounded down to 16 bytes
+   typedef T vec __attribute__((ext_vector_type(VK)));
+   const int r = lane & 15, kq = lane >> 4, ntile = (n + 15) >> 4;
+   const int lgt = ntile <= 1 ? 0 : ntile <= 2 ? 1 : 2, sp = wave >> lgt, nsp = 4 >> lgt;
+   const int nlo = n & ~(VK - 1), nst = (m - nlo + RS - 1) / RS;
+   vec ap[4];
+   auto load_rows = [&](int tile, int st) {
+      const int j = tile * 16 + r;
+      const uint32_t vo = j < n ? (uint32_t)(nlo + kq * VK + j * ld) * ES : kOut;
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+         if (st + u * nsp < nst) {
+            const uint32_t so = (uint32_t)((st + u * nsp) * RS) * ES;
+            const auto raw = __builtin_amdgcn_raw_buffer_load_b128(frs, (int)vo, (int)so, 0);
+            __builtin_memcpy(&ap[u], &raw, 16);
+         }
+   };
+   const int tile0 = wave & ((1 << lgt) - 1);
+   if constexpr (BWD) {
+      if (q > 0) load_rows(tile0, sp);
+   } else {
+      few_load(a, mrs, vo1, (uint32_t)n * ES, 0, K1);
+   }
+   // the front's x: backward every row from the solution; forward b on the
+   // pivot rows, zero below, then the children's contribution rows in list order
+#pragma unroll
+   for (int c = 0; c < NR; ++c) {
+      double v = 0.0;
+      if (gi >= 0 && c < nc) v = BWD ? xsol[gi + (int64_t)(c0 + c) * ldsol] : b[gi + (int64_t)(c0 + c) * ldb];
+      if (tid < kNB) x1[c][tid] = tid < n ? v : 0.0;
+      x2[c][tid] = 0.0;
+      if (tid < kNB) ys[c][tid] = 0.0;
+      if (BWD && q > 0) {
+         __syncthreads();
+         if (tid >= n && tid < m) x2[c][tid - n] = v;
+      }
+   }
+   if constexpr (!BWD) {
+      int cm = 0, ch = nd.first_child;
+      double cx[NR];
+      auto load_child = [&](const NodeDesc& cn) {
+         if (tid < cn.m - cn.n) {
+            const double* p = xloc + cn.solve_off * nrhs + (int64_t)c0 * cn.m + cn.n + tid;
+            cm = cmap[cn.cmap_off + tid];
+#pragma unroll
+            for (int c = 0; c < NR; ++c) cx[c] = c < nc ? p[(int64_t)c * cn.m] : 0.0;
+         } else {
+            cm = -1;
+         }
+      };
+      int next = -1;
+      if (ch != -1) {
+         const NodeDesc cn = nodes[ch];
+         load_child(cn);
+         next = cn.next_child;
+      }
+      while (ch != -1) {
+         const int row = cm;
+         double val[NR];
+#pragma unroll
+         for (int c = 0; c < NR; ++c) val[c] = cx[c];
+         ch = next;
+         if (ch != -1) {
+            const NodeDesc cn = nodes[ch];
+            load_child(cn);
+            next = cn.next_child;
+         }
+         __syncthreads();
+         if (row >= 0)
+#pragma unroll
+            for (int c = 0; c < NR; ++c) (row < n ? x1[c][row] : x2[c][row - n]) += val[c];
+      }
+   }
+   __syncthreads();
+   if constexpr (BWD) {
+      if (q > 0) {  // x[0:n] -= L21^T x[n:m]
+         for (int tile = tile0; tile < ntile; tile += 4) {
+            double acc[NR];
+#pragma unroll
+            for (int c = 0; c < NR; ++c) acc[c] = 0.0;
+            for (int st = sp; st < nst; st += 4 * nsp) {
+               if (tile != tile0 || st != sp) load_rows(tile, st);
+#pragma unroll
+               for (int u = 0; u < 4; ++u)
+                  if (st + u * nsp < nst)
+#pragma unroll
+                     for (int e = 0; e < VK; ++e) {
+                        const int row = nlo - n + (st + u * nsp) * RS + kq * VK + e;
+                        const bool in = row >= 0 && row < q;
+                        const double l = in ? (double)ap[u][e] : 0.0;
+#pragma unroll
+                        for (int c = 0; c < NR; ++c) acc[c] = fma(l, x2[c][in ? row : 2 * kNB - 1], acc[c]);
+                     }
+            }
+#pragma unroll
+            for (int c = 0; c < NR; ++c) {
+               acc[c] += __shfl_xor(acc[c], 16);
+               acc[c] += __shfl_xor(acc[c], 32);
+               if (lane < 16) red[c][sp * (16 << lgt) + tile * 16 + r] = acc[c];
+            }
+         }
+      }
+      few_load(a, mrs, vo1, (uint32_t)n * ES, 0, K1);
+      if (q > 0) {
+         __syncthreads();
+         if (tid < n)
+#pragma unroll
+            for (int c = 0; c < NR; ++c) {
+               double sum = red[c][tid];
+               for (int g = 1; g < nsp; ++g) sum += red[c][g * (16 << lgt) + tid];
+               x1[c][tid] -= sum;
+            }
+         __syncthreads();
+      }
+   }
+   double acc[NR];
+#pragma unroll
+   for (int c = 0; c < NR; ++c) acc[c] = 0.0;
+   few_rows<T, NR>(a, mrs, vo1, (uint32_t)n * ES, K1, &x1[0][g1 * K1], kNB, acc);
+   const int lgq = lg_rows(q), K2 = group_cols(lgq), i2 = tid & ((1 << lgq) - 1), g2 = tid >> lgq;
+   const uint32_t vo2 = i2 < q ? (uint32_t)(i2 + g2 * K2 * ld) * ES : kOut;
+   if (!BWD && q > 0) few_load(a, frs, vo2, (uint32_t)ld * ES, 0, K2);
+#pragma unroll
+   for (int c = 0; c < NR; ++c) red[c][tid] = acc[c];
+   __syncthreads();
+   if (tid < n)
+#pragma unroll
+      for (int c = 0; c < NR; ++c) {
+         double y = 0.0;
+         for (int g = 0; g < (256 >> lgp); ++g) y += red[c][(g << lgp) + tid];
+         if (!BWD) ys[c][tid] = y;
+         if (c < nc) xsol[gi + (int64_t)(c0 + c) * ldsol] = y;
+      }
+   if (BWD || q == 0) return;
+   __syncthreads();
+   // x[n:m] -= L21 y
+#pragma unroll
+   for (int c = 0; c < NR; ++c) acc[c] = 0.0;
+   few_rows<T, NR>(a, frs, vo2, (uint32_t)ld * ES, K2, &ys[0][g2 * K2], kNB, acc);
+#pragma unroll
+   for (int c = 0; c < NR; ++c) red[c][tid] = acc[c];
+   __syncthreads();
+   if (tid < q)
+#pragma unroll
+      for (int c = 0; c < NR; ++c)
+         if (c < nc) {
+            double sum = 0.0;
+            for (int g = 0; g < (256 >> lgq); ++g) sum += red[c][(g << lgq) + tid];
+            xloc[nd.solve_off * nrhs + (int64_t)(c0 + c) * m + n + tid] = x2[c][tid] - sum;
+         }
 }
 
 // Backward contribution-block update split over row chunks: task (node,

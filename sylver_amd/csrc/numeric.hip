@@ -1488,15 +1488,28 @@ void run_solve_program(const DevicePlan* P, DeviceFactors* F, const std::vector<
                k_bwd_cbp<T><<<g, bl, 0, s>>>(tk, P->d_nodes, arena, xsol, n, P->d_rlist, F->d_part_cb, nrhs);
             break;
          case L_FSMALL:
-            k_solve_small<T, false><<<g, bl, small_lds(L), s>>>(P->d_nlistv + L.off, P->d_nodes, arena, dinv,
-                                                                P->d_rlist, F->d_xloc, xsol, n, nrhs, b, n,
-                                                                P->d_cmap, (L.smax_m + 15) & ~15);
+         case L_BSMALL: {
+            const bool bwd = L.kind == L_BSMALL;
+            const ChainShape c = small_shape(nrhs, L.count);
+            auto small = [&](auto kernel, size_t lds, auto... rest) {
+               const dim3 gs = c.width < 16 ? dim3(L.count * c.grid) : dim3(L.count, c.grid);
+               kernel<<<gs, bl, lds, s>>>(P->d_nlistv + L.off, P->d_nodes, arena, bwd ? dinvT : dinv, P->d_rlist,
+                                         F->d_xloc, xsol, n, nrhs, bwd ? nullptr : b, bwd ? 0 : n, P->d_cmap, rest...,
+                                         c.grid);
+            };
+            const int mrows = (L.smax_m + 15) & ~15;
+            if (c.width == 1)
+               bwd ? small(k_solve_small_few<T, true, 1>, 0) : small(k_solve_small_few<T, false, 1>, 0);
+            else if (c.width == 2)
+               bwd ? small(k_solve_small_few<T, true, 2>, 0) : small(k_solve_small_few<T, false, 2>, 0);
+            else if (c.width == 4)
+               bwd ? small(k_solve_small_few<T, true, 4>, 0) : small(k_solve_small_few<T, false, 4>, 0);
+            else if (bwd)
+               small(k_solve_small<T, true>, small_lds(L), mrows);
+            else
+               small(k_solve_small<T, false>, small_lds(L), mrows);
             break;
-         case L_BSMALL:
-            k_solve_small<T, true><<<g, bl, small_lds(L), s>>>(P->d_nlistv + L.off, P->d_nodes, arena, dinvT,
-                                                               P->d_rlist, F->d_xloc, xsol, n, nrhs, nullptr, 0,
-                                                               P->d_cmap, (L.smax_m + 15) & ~15);
-            break;
+         }
          case L_BRED:
             if (L.count > 0) k_bwd_cbr<<<g, bl, 0, s>>>(tk, P->d_nodes, F->d_part_cb, F->d_xloc, nrhs);
             break;

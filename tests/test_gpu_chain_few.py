@@ -1,7 +1,8 @@
-"""The chained solve's kernels by number of right-hand sides: vector sums for
-one column, chunks of two up to eight, 16-column MFMA tiles beyond, the chunks
-side by side. Dense fronts around the edges of the 128-row blocks, and a 3D
-grid, whose fronts have children and contribution blocks."""
+"""The solve kernels by number of right-hand sides: vector sums in chunks up
+to eight columns, 16-column MFMA tiles beyond, the chunks side by side. Dense
+fronts around the edges of the 128-row blocks (the chained launch) and of the
+16 .. 128 rows that threads are dealt by (the small fronts), and grids, whose
+fronts have children and contribution blocks."""
 import numpy as np
 import pytest
 
@@ -23,7 +24,7 @@ def _solver(S, A, prec):
 
 
 @pytest.mark.parametrize("prec,u", [("fp64", 2.0 ** -53), ("fp32", 2.0 ** -24)])
-@pytest.mark.parametrize("n", [129, 255, 256, 257, 400])
+@pytest.mark.parametrize("n", [1, 15, 17, 32, 33, 65, 127, 128, 129, 255, 256, 257, 400])
 def test_dense_front_all_widths(S, O, gpu, n, prec, u):
     """n I + U[-1, 1] (condition below 2): the factorization is wrong by at
     most (n + 1) u |L| |L^T|, each triangular solve by n u |L|, so 8 n u
@@ -63,3 +64,23 @@ def test_grid_columns_alike(S, O, gpu, prec):
         assert max(errs) <= 1e-14, errs
     else:
         assert max(errs) <= 8 * min(errs), errs
+
+
+@pytest.mark.parametrize("nx,ny,nz", [(31, 17, 1), (64, 61, 1), (9, 8, 7)])
+def test_ragged_small_fronts(S, O, gpu, nx, ny, nz):
+    """Small fronts of many shapes (odd pivot counts, so that the rows below
+    them start off 16 bytes), FP64: the bar of the other FP64 solves."""
+    rng = np.random.default_rng(nx)
+    g = np.arange(nx * ny * nz).reshape(nz, ny, nx)
+    pairs = [(g[:, :, :-1], g[:, :, 1:]), (g[:, :-1], g[:, 1:]), (g[:-1], g[1:])]
+    lo = np.concatenate([p.ravel() for p, _ in pairs] + [g.ravel()])
+    hi = np.concatenate([p.ravel() for _, p in pairs] + [g.ravel()])
+    val = np.where(lo == hi, 7.0, -rng.uniform(0.5, 1.0, len(lo)))
+    order = np.lexsort((hi, lo))
+    A = M._from_coo_lower(g.size, hi[order], lo[order], val[order])
+    d = _solver(S, A, "fp64")
+    b = M.random_rhs(A.n, max(NRHS), seed=6)
+    for k in NRHS:
+        y = b[:, :k].copy(order="F")
+        assert S.spldlt_solve(y, d.akeep, d.fkeep, options=d.options).flag == 0
+        assert O.bwd_err(A, y, np.asfortranarray(b[:, :k])) <= 1e-14, k
