@@ -854,7 +854,7 @@ static __global__ __launch_bounds__(kThreads) void k_app_front(const int* __rest
 //   k_lp_finish  passed count, L11, D^{-1}, failed-column list;
 //   k_lp_update  restore of the failed columns and update of every
 //                uneliminated fully-summed column (lower triangle, mirrored),
-//                128 x 128 tiles, one FMA chain per entry in pivot order.
+//                64 x 64 tiles, one FMA chain per entry in pivot order.
 // Then k_lp_np / k_lp_pgather / k_lp_pscatter (permute_failed) and k_lp_tail
 // (the second pass). Every entry goes through the same arithmetic, in the
 // same order, as in k_app_front, so the two give identical factors.
@@ -1173,7 +1173,7 @@ __device__ __forceinline__ bool lp_keep(int mode, int rpos, int spos, int nf, in
 // columns and U followed by rows n .. m - 1 for rows, gets
 // x -= L[r, c0 + p] (D L[s, :])_p for p = 0 .. npass - 1 in that order; the
 // fully-summed part is mirrored. Entries of the failed block columns start
-// from the backup (the restore). 128 x 128 tiles, 8 x 8 entries per thread,
+// from the backup (the restore). 64 x 64 tiles, 4 x 4 entries per thread,
 // tiles taken in turn by a grid of any size.
 static __global__ __launch_bounds__(kThreads) void k_lp_update(int node, int c0, int par, int mode,
                                                         const IndefDesc* __restrict__ nodes,
